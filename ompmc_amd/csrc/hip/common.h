@@ -30,103 +30,99 @@ constexpr int MAX_PHANTOMS = 16;     // resident phantoms per context
 // RANMAR numbers ompMC uses.  A secondary's key is the Philox block
 // (parent ctr, 1, 0, 0) under the parent key, taken after the interaction's
 // last draw, so every history is independent of processing order.
+//
+// One round: the two 32x32 products as 64-bit multiplications, which the
+// compiler turns into one v_mad_u64_u32 each instead of a v_mul_lo and a
+// v_mul_hi (all of them quarter rate).
+__device__ __forceinline__ void philox_round(uint32_t &c0, uint32_t &c1, uint32_t &c2, uint32_t &c3, uint32_t k0,
+                                             uint32_t k1)
+{
+    const uint64_t p0 = (uint64_t)0xD2511F53u * c0, p1 = (uint64_t)0xCD9E8D57u * c2;
+    const uint32_t n0 = (uint32_t)(p1 >> 32) ^ c1 ^ k0;
+    const uint32_t n2 = (uint32_t)(p0 >> 32) ^ c3 ^ k1;
+    c0 = n0; c1 = (uint32_t)p1; c2 = n2; c3 = (uint32_t)p0;
+}
+
 __device__ __forceinline__ void philox10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3,
                                          uint32_t k0, uint32_t k1, uint32_t out[4])
 {
 #pragma unroll
     for (int r = 0; r < 10; ++r) {
         if (r) { k0 += 0x9E3779B9u; k1 += 0xBB67AE85u; }
-        uint32_t lo0 = 0xD2511F53u * c0, hi0 = __umulhi(0xD2511F53u, c0);
-        uint32_t lo1 = 0xCD9E8D57u * c2, hi1 = __umulhi(0xCD9E8D57u, c2);
-        uint32_t n0 = hi1 ^ c1 ^ k0;
-        uint32_t n2 = hi0 ^ c3 ^ k1;
-        c0 = n0; c1 = lo1; c2 = n2; c3 = lo0;
+        philox_round(c0, c1, c2, c3, k0, k1);
     }
     out[0] = c0; out[1] = c1; out[2] = c2; out[3] = c3;
 }
 
 // The same function with its rounds kept as a loop: for the rare paths
 // inlined at every draw site (a block the ring does not hold, a secondary's
-// key).  Unrolled there, Philox was half of the charged-particle kernel's
-// instructions (about a hundred inlined copies), far more code than the
-// instruction cache a CU pair shares holds.
+// key), where ten unrolled rounds would be most of the kernel's code.
 __device__ __forceinline__ void philox10_rolled(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3,
                                                 uint32_t k0, uint32_t k1, uint32_t out[4])
 {
 #pragma unroll 1
     for (int r = 0; r < 10; ++r) {
-        uint32_t lo0 = 0xD2511F53u * c0, hi0 = __umulhi(0xD2511F53u, c0);
-        uint32_t lo1 = 0xCD9E8D57u * c2, hi1 = __umulhi(0xCD9E8D57u, c2);
-        uint32_t n0 = hi1 ^ c1 ^ k0;
-        uint32_t n2 = hi0 ^ c3 ^ k1;
-        c0 = n0; c1 = lo1; c2 = n2; c3 = lo0;
+        philox_round(c0, c1, c2, c3, k0, k1);
         k0 += 0x9E3779B9u; k1 += 0xBB67AE85u;
     }
     out[0] = c0; out[1] = c1; out[2] = c2; out[3] = c3;
 }
 
-// Look-ahead of a lane's stream in LDS: RNG_RING Philox blocks per lane,
-// block b in slot b % RNG_RING of the lane's column.  A transport kernel
-// that uses it tops the ring up where the wavefront's live lanes are
-// converged (the head of each trip), so the draw sites read 16 bytes from
-// LDS instead of running Philox in whichever few lanes crossed a block
-// boundary there.  The words and their order are those of the stream
-// itself.  The ring is the launch's dynamic LDS (RNG_RING_BYTES), so only
-// the launches that top it up pay for it in occupancy.
+// The uniform of a Philox word: (w >> 8) * 2^-24, exact in FP32.
+__device__ __forceinline__ float philox_uniform(uint32_t w) { return (float)(w >> 8) * (1.0f / 16777216.0f); }
+
+// Look-ahead of a lane's stream in LDS: RNG_RING Philox blocks per lane as
+// ready uniforms, draw d in row d % (4 * RNG_RING) of the lane's column (rows
+// are a block's threads wide, so any mix of rows is free of bank conflicts).
+// A draw is then one 4-byte LDS read behind a wavefront-wide test that the
+// ring holds it: about 8 instructions.  Holding the current block's four
+// words in registers instead, as this engine did before, took about 50 per
+// draw: the compiler carried the words, the block number and the ring's end
+// through every divergent region of some fifty draw sites (2200 of the FP32
+// charged-particle kernel's 13400 vector instructions were such copies).
+// ring_fill() tops the rings of a wavefront up where its lanes are converged
+// (the head of each trip).  The words and their order are those of the stream
+// itself.  The ring is the launch's dynamic LDS (RNG_RING_BYTES).
 constexpr uint32_t RNG_RING = 8;
 constexpr int RNG_LANES = 256;           // threads per transport block
-constexpr size_t RNG_RING_BYTES = (size_t)RNG_RING * RNG_LANES * sizeof(uint4);
-extern __shared__ uint4 rng_ring[];      // [RNG_RING][RNG_LANES]
+constexpr size_t RNG_RING_BYTES = (size_t)RNG_RING * 4 * RNG_LANES * sizeof(float);
+extern __shared__ float rng_ring[];      // [4 * RNG_RING][RNG_LANES]
+
+// Computes block b of stream (k0, k1) into the ring column `col`.
+template <bool ROLLED>
+__device__ __forceinline__ void ring_block(uint32_t b, uint32_t k0, uint32_t k1, uint32_t col)
+{
+    uint32_t o[4];
+    if (ROLLED) philox10_rolled(b, 0u, 0u, 0u, k0, k1, o);
+    else philox10(b, 0u, 0u, 0u, k0, k1, o);
+    float *r = rng_ring + (b % RNG_RING) * (4 * RNG_LANES) + col;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i * RNG_LANES] = philox_uniform(o[i]);
+}
 
 struct Rng {
     uint32_t k0, k1, ctr;
-    uint32_t blk;            // block held in w[] (0xffffffff = none)
-    uint32_t w0, w1, w2, w3;
-    uint32_t tail;           // blocks in [ctr >> 2, tail) are in this thread's LDS ring
+    uint32_t tail;           // draws [ctr, tail) are in this thread's ring column (multiple of 4)
 
-    // No cached block, nothing in the ring: every block is computed at the
-    // draw (secondaries, fresh primaries, particles read from a queue).
-    // Only the stream of the particle a transport lane owns is topped up,
-    // so only that stream ever finds blocks in the thread's ring column.
-    __device__ __forceinline__ void reset_cache() { blk = 0xffffffffu; tail = 0u; }
+    // Nothing in the ring (secondaries, particles read from a queue).  Only
+    // the stream of the particle a transport lane owns is drawn from, so the
+    // thread's column holds that stream only.
+    __device__ __forceinline__ void reset_cache() { tail = 0u; }
 
-    // Fill the thread's ring up to `depth` blocks ahead of the next draw
-    // (transport kernels, for the stream of the lane's own particle).
-    __device__ __forceinline__ void top_up(uint32_t depth)
+    // Next uniform.  The test is taken by the wavefront's active lanes
+    // together (a scalar branch); a stream that ran past its ring computes
+    // its next block on the spot.
+    __device__ __forceinline__ float next()
     {
-        const uint32_t cur = ctr >> 2;
-        if (tail < cur) tail = cur;
-        while (tail < cur + depth) {
-            uint32_t o[4];
-            philox10(tail, 0u, 0u, 0u, k0, k1, o);
-            rng_ring[(tail % RNG_RING) * RNG_LANES + threadIdx.x] = make_uint4(o[0], o[1], o[2], o[3]);
-            tail++;
-        }
-    }
-
-    __device__ __forceinline__ uint32_t next_u24()
-    {
-        uint32_t b = ctr >> 2;
-        if (b != blk) {
-            if (b < tail) {
-                const uint4 v = rng_ring[(b % RNG_RING) * RNG_LANES + threadIdx.x];
-                w0 = v.x; w1 = v.y; w2 = v.z; w3 = v.w;
-            } else {
-                uint32_t o[4];
-                philox10_rolled(b, 0u, 0u, 0u, k0, k1, o);
-                w0 = o[0]; w1 = o[1]; w2 = o[2]; w3 = o[3];
-                tail = b + 1;
+        const uint32_t c = ctr;
+        if (__ballot(c >= tail) != 0) {
+            if (c >= tail) {
+                ring_block<true>(c >> 2, k0, k1, threadIdx.x);
+                tail = (c & ~3u) + 4u;
             }
-            blk = b;
         }
-        // word (ctr & 3) of the block by two selects on its bits (a select
-        // chain on the whole value becomes an indexed private array)
-        const uint32_t s = ctr & 3u;
-        const uint32_t even = (s & 2u) ? w2 : w0;
-        const uint32_t odd = (s & 2u) ? w3 : w1;
-        const uint32_t w = (s & 1u) ? odd : even;
-        ctr++;
-        return w >> 8;
+        ctr = c + 1u;
+        return rng_ring[(c % (4 * RNG_RING)) * RNG_LANES + threadIdx.x];
     }
     // Key of a secondary: the Philox block (ctr, tag, 0, 0) under this key.
     // Interactions use tag 1 for the particles they create; tag 2 is for a
@@ -140,11 +136,23 @@ struct Rng {
     }
 };
 
+// A stream read in order by one thread without a ring (the source kernel).
+struct SeqRng {
+    uint32_t k0, k1, ctr;
+    uint32_t w[4];
+
+    __device__ __forceinline__ float next()
+    {
+        if ((ctr & 3u) == 0u) philox10(ctr >> 2, 0u, 0u, 0u, k0, k1, w);
+        const float even = philox_uniform((ctr & 2u) ? w[2] : w[0]), odd = philox_uniform((ctr & 2u) ? w[3] : w[1]);
+        const float x = (ctr & 1u) ? odd : even;
+        ctr++;
+        return x;
+    }
+};
+
 // next uniform of a particle stream, in [0,1) with 24-bit granularity
-template <typename R> __device__ __forceinline__ R urand(Rng &r)
-{
-    return (R)r.next_u24() * (R)(1.0 / 16777216.0);
-}
+template <typename R, typename S> __device__ __forceinline__ R urand(S &r) { return (R)r.next(); }
 
 __device__ __forceinline__ void primary_key(uint32_t s0, uint32_t s1, uint64_t hid, uint32_t &k0, uint32_t &k1)
 {
@@ -182,6 +190,68 @@ __device__ __forceinline__ void wave_max_to(uint32_t *p, uint32_t v)
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, o));
     if (lane_id() == 0 && v) atomicMax(p, v);
+}
+
+// Tops up the Philox rings of a wavefront's live lanes; every lane of the
+// wavefront calls it, converged (`mask` is the ballot of `live`).
+//
+// With at most half of the lanes live, the idle lanes compute blocks too:
+// each live lane gets 2, 4 or 8 consecutive lanes of the wavefront, which
+// share its missing blocks (8 helpers do all of them in one pass).  A lone
+// particle's trip spent a fifth of its time on four or five passes of one
+// lane each.
+//
+// A fuller wavefront computes one block per lane and pass, as long as
+// RNG_FILL_LANES lanes have room for one or a lane holds fewer than
+// RNG_FILL_MIN: the few lanes that drew most in the last trip catch up over
+// the next ones instead of costing the wavefront a pass each.
+#ifndef OMC_RNG_FILL_LANES
+#define OMC_RNG_FILL_LANES 24
+#endif
+#ifndef OMC_RNG_FILL_MIN
+#define OMC_RNG_FILL_MIN 6
+#endif
+__device__ __forceinline__ void ring_fill(Rng &r, bool live, uint64_t mask)
+{
+    const uint32_t cur = r.ctr >> 2;
+    uint32_t tb = max(r.tail >> 2, cur);                    // first block not in the ring
+    uint32_t room = live ? cur + RNG_RING - tb : 0u;
+    const int nlive = __popcll(mask);
+    if (nlive <= 32) {
+        const int sh = nlive <= 8 ? 3 : nlive <= 16 ? 2 : 1;
+        const int lane = lane_id();
+        const int rank = (int)lanes_below(mask);            // among the live lanes
+        // lane i learns the live lane of rank i: a permutation, live lanes first
+        const int at = live ? rank : nlive + lane - rank;
+        const int of_rank = __builtin_amdgcn_ds_permute(at << 2, lane);
+        const int own = __builtin_amdgcn_ds_bpermute((lane >> sh) << 2, of_rank);
+        const uint32_t k0 = (uint32_t)__builtin_amdgcn_ds_bpermute(own << 2, (int)r.k0);
+        const uint32_t k1 = (uint32_t)__builtin_amdgcn_ds_bpermute(own << 2, (int)r.k1);
+        const uint32_t first = (uint32_t)__builtin_amdgcn_ds_bpermute(own << 2, (int)tb);
+        // (every lane takes part in the exchange: a lane that is masked off
+        // has no value to give)
+        const uint32_t want = (uint32_t)__builtin_amdgcn_ds_bpermute(own << 2, (int)room);
+        const uint32_t n = (lane >> sh) < nlive ? want : 0u;
+        const uint32_t col = (threadIdx.x & ~63u) + (uint32_t)own;
+        for (uint32_t j = (uint32_t)lane & ((1u << sh) - 1u); __ballot(j < n) != 0; j += 1u << sh)
+            if (j < n) ring_block<false>(first + j, k0, k1, col);
+        tb += room;
+    } else {
+        while (__popcll(__ballot(room != 0u)) >= OMC_RNG_FILL_LANES ||
+               __ballot(room > RNG_RING - OMC_RNG_FILL_MIN) != 0) {
+            if (room) {
+                ring_block<false>(tb, r.k0, r.k1, threadIdx.x);
+                tb++;
+                room--;
+            }
+        }
+    }
+    if (live) r.tail = tb << 2;
+    // the helpers' writes come before the owners' reads: LDS executes a
+    // wavefront's accesses in order, and this keeps the compiler to it
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // ------------------------------------------------------------- layouts ----

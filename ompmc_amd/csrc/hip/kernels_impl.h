@@ -50,13 +50,13 @@ __global__ void __launch_bounds__(256) k_source(const DevJob *jobs, const DevPha
     Particle<R> p;
     p.job = (uint32_t)job;
     p.hist = (uint32_t)h;
-    primary_key(J.s0, J.s1, J.hist0 + h, p.rng.k0, p.rng.k1);
-    p.rng.ctr = 0u;
-    p.rng.reset_cache();
+    SeqRng rng;
+    primary_key(J.s0, J.s1, J.hist0 + h, rng.k0, rng.k1);
+    rng.ctr = 0u;
     p.iq = J.charge;
     R ein;
     if (J.spectrum) {
-        R r1 = urand<R>(p.rng), r2 = urand<R>(p.rng);
+        R r1 = urand<R>(rng), r2 = urand<R>(rng);
         int k = (int)fmin(J.deltak * (double)r1, J.deltak - 1.0);
         ein = (R)J.cdf1[k] + r2 * (R)J.cdf2[k];
     } else {
@@ -75,11 +75,11 @@ __global__ void __launch_bounds__(256) k_source(const DevJob *jobs, const DevPha
         } else {
             R fw, r3;
             do {
-                r3 = urand<R>(p.rng);
+                r3 = urand<R>(rng);
                 p.x = r3 * (R)J.xsize + (R)J.xinl;
-                r3 = urand<R>(p.rng);
+                r3 = urand<R>(rng);
                 p.y = r3 * (R)J.ysize + (R)J.yinl;
-                r3 = urand<R>(p.rng);
+                r3 = urand<R>(rng);
                 rxyz = m_sqrt(ssd * ssd + p.x * p.x + p.y * p.y);
                 p.w = ssd / rxyz;
                 fw = p.w * p.w * p.w;
@@ -93,7 +93,7 @@ __global__ void __launch_bounds__(256) k_source(const DevJob *jobs, const DevPha
         iy = J.ysize == 0.0 ? J.iyinl : scan_bounds<R>(g.yb, J.iyinl - 1, g.jsize - 1, p.y);
         p.ir = 1 + ix + iy * g.isize;
     } else {
-        R r1 = urand<R>(p.rng), r2 = urand<R>(p.rng);
+        R r1 = urand<R>(rng), r2 = urand<R>(rng);
         R xiso = r1 * (R)J.side1[0] + r2 * (R)J.side2[0] + (R)J.corner[0];
         R yiso = r1 * (R)J.side1[1] + r2 * (R)J.side2[1] + (R)J.corner[1];
         R ziso = r1 * (R)J.side1[2] + r2 * (R)J.side2[2] + (R)J.corner[2];
@@ -123,6 +123,8 @@ __global__ void __launch_bounds__(256) k_source(const DevJob *jobs, const DevPha
         const int iz = scan_bounds<R>(g.zb, 0, g.ksize - 1, p.z);
         p.ir = 1 + ix + iy * g.isize + iz * g.isize * g.jsize;
     }
+    p.rng.k0 = rng.k0; p.rng.k1 = rng.k1; p.rng.ctr = rng.ctr;
+    p.rng.reset_cache();
     push<R>(p.iq == 0 ? qp : qe, p, st);
 }
 
@@ -138,13 +140,13 @@ void Launch<R>::source(const DevJob *jobs, const DevPhantom<R> *ph, const Source
 template <typename R>
 void Launch<R>::photon(const KArgs<R> &a, int grid, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_photon<R>, dim3(grid), dim3(RNG_LANES), OMC_RNG_DEPTH_P ? RNG_RING_BYTES : 0, s, a);
+    hipLaunchKernelGGL(k_photon<R>, dim3(grid), dim3(RNG_LANES), RNG_RING_BYTES, s, a);
 }
 
 template <typename R>
 void Launch<R>::electron(const KArgs<R> &a, int grid, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_electron<R>, dim3(grid), dim3(RNG_LANES), OMC_RNG_DEPTH_E ? RNG_RING_BYTES : 0, s, a);
+    hipLaunchKernelGGL(k_electron<R>, dim3(grid), dim3(RNG_LANES), RNG_RING_BYTES, s, a);
 }
 
 // The transport's math functions (m_log ... m_pow in the precision R, as

@@ -1036,18 +1036,6 @@ __device__ __forceinline__ int electron_iteration(const KArgs<R> &A, Particle<R>
 #ifndef OMC_WAVES_E64
 #define OMC_WAVES_E64 2
 #endif
-// Philox blocks each lane keeps ready in its LDS ring at the head of a trip
-// (at most RNG_RING; 0 = no ring).  An electron trip draws about 15
-// numbers; a photon trip draws a few and its kernel waits on voxel loads,
-// so it keeps the occupancy the ring's LDS would cost.
-#ifndef OMC_RNG_DEPTH_E
-#define OMC_RNG_DEPTH_E 8
-#endif
-#ifndef OMC_RNG_DEPTH_P
-#define OMC_RNG_DEPTH_P 0
-#endif
-static_assert(OMC_RNG_DEPTH_E <= RNG_RING && OMC_RNG_DEPTH_P <= RNG_RING, "ring depth");
-
 template <typename R> struct Waves;
 template <> struct Waves<float> { static constexpr int photon = OMC_WAVES_P32, electron = OMC_WAVES_E32; };
 template <> struct Waves<double> { static constexpr int photon = OMC_WAVES_P64, electron = OMC_WAVES_E64; };
@@ -1102,8 +1090,8 @@ __global__ void __launch_bounds__(256, Waves<R>::photon) k_photon(KArgs<R> A)
         // none can step; until then the waiting lanes sit out the steps
         const uint32_t nev = (uint32_t)__popcll(__ballot(alive && s.phase != 1));
         const bool events = nev * A.event_div >= nlive || nev == nlive;
+        ring_fill(p.rng, alive, live);
         if (alive && (s.phase == 1 || events)) {
-            if (OMC_RNG_DEPTH_P) p.rng.top_up(OMC_RNG_DEPTH_P);
             if (s.phase != 1)
                 alive = photon_event<R>(A, p, s, G, sc);
             else if (A.woodcock && G.g->wc.mu && s.split == 0u)
@@ -1178,8 +1166,8 @@ __global__ void __launch_bounds__(256, Waves<R>::electron) k_electron(KArgs<R> A
         if (live == 0) break;
         const bool drain =
             in_end >= A.drain_min && __ballot(exhausted) != 0 && (uint32_t)__popcll(live) <= A.drain_lanes;
+        ring_fill(p.rng, alive, live);
         if (alive) {
-            p.rng.top_up(OMC_RNG_DEPTH_E);
             int r = electron_iteration<R>(A, p, s, G, sc, nsteps, ncross);
             ++trips;
             ++here;
