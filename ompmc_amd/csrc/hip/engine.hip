@@ -93,6 +93,22 @@ constexpr int64_t DEFAULT_CHUNK = 1 << 22;
 // cause not yet found, so the count is held near the range that has run.
 constexpr int64_t MAX_SPLIT_INFLIGHT = 16;
 constexpr uint32_t DEFAULT_YIELD_TRIPS = 4096;
+// A launch whose input is below the drain threshold (it cannot fill the
+// device) hands its particles on after this many trips: the photons that its
+// charged particles have made by then are followed while its longest tracks
+// go on, instead of after them, and the tracks left are spread over the
+// device again.  A generation costs about 0.2 ms, as much as 40 trips of a
+// lone particle.  One 2e4-history beamlet request on the patient phantom, FP32
+// / FP64: 18.9 / 27.5 ms at 4096 trips, 18.7 / 30.7 at 512, 20.2 / 34.5 at
+// 256; 1e6 photons on the graded 61^3 grid, FP32, 56 / 46 / 47 ms.
+constexpr uint32_t SMALL_YIELD_TRIPS = 512;
+// Wavefronts per SIMD over which a small launch's particles are spread
+// (lanes_used).  A 1e3-photon FP64 call on the 40^3 water cube takes 8.7 ms
+// with 64 particles to a wavefront, 5.1-5.3 ms spread over 1, 2 or 4 per
+// SIMD; the FP32 beamlet request 22.5 ms against 18.7; with 4 per SIMD the
+// wavefronts of larger inputs (2e5 electrons, 1e6 photons) slow each other
+// down (5e6 FP64 slab histories 120 ms against 109 at 2).
+constexpr int SPREAD_WAVES = 2;
 // Drain compaction: once a launch's input is used up, a wavefront with at
 // most 32 live lanes hands its particles (after 16 trips in the launch) to
 // the next launch, which packs them into full wavefronts (slab sweep: FP32
@@ -1023,6 +1039,14 @@ static int pull_segments(omc_dev_ctx *c, int pi, int64_t room, uint32_t &injP, u
     return nseg;
 }
 
+// Blocks of a transport launch over at most n particles.
+static int transport_grid(const omc_dev_ctx *c, int64_t n)
+{
+    const int64_t full = (n + RNG_LANES - 1) / RNG_LANES, wide = (int64_t)c->cus * SPREAD_WAVES;
+    const int64_t one = (n + RNG_LANES / 64 - 1) / (RNG_LANES / 64);      // one particle per wavefront
+    return (int)std::max<int64_t>(1, std::min<int64_t>((int64_t)c->cus * 8, std::max(full, std::min(one, wide))));
+}
+
 template <typename R> static int launch_generation(omc_dev_ctx *c, int pi)
 {
     Pipe &P = c->pipes[pi];
@@ -1057,13 +1081,13 @@ template <typename R> static int launch_generation(omc_dev_ctx *c, int pi)
     A.qp = queue_view<R>(c, P, nxt);
     A.status = P.d_status;
     A.yield_trips = c->yield_trips;
+    A.yield_small = SMALL_YIELD_TRIPS;
     A.drain_lanes = c->drain_lanes;
     A.drain_trips = c->drain_trips;
     A.drain_min = (uint32_t)std::min<int64_t>(c->drain_min, UINT32_MAX);
     A.event_div = c->event_div;
     A.fetch_min = c->fetch_min;
     A.woodcock = c->woodcock ? 1u : 0u;
-    const int max_grid = c->cus * 8;
     P.had_ph = inP > 0;
     P.in_e = inE;
     if (P.had_ph) {
@@ -1073,7 +1097,7 @@ template <typename R> static int launch_generation(omc_dev_ctx *c, int pi)
         A.fetch = P.d_counts + 4;
         A.longest = P.d_counts + 7;
         HIPCHK(hipEventRecord(P.ev_ph0, s));
-        Launch<R>::photon(A, (int)std::min<int64_t>(max_grid, ((int64_t)inP + 255) / 256), s);
+        Launch<R>::photon(A, transport_grid(c, inP), s);
         HIPCHK(hipEventRecord(P.ev_ph1, s));
     }
     P.had_el = inE > 0 || inP > 0;
@@ -1094,7 +1118,7 @@ template <typename R> static int launch_generation(omc_dev_ctx *c, int pi)
             Launch<R>::sort_charged(qec, P.d_sort, sorted, s);
             A.qin = sorted;
         }
-        Launch<R>::electron(A, (int)std::min<int64_t>(max_grid, ((int64_t)inE + 2 * (int64_t)inP + 255) / 256), s);
+        Launch<R>::electron(A, transport_grid(c, (int64_t)inE + 2 * (int64_t)inP), s);
         HIPCHK(hipEventRecord(P.ev_el1, s));
     }
     HIPCHK(hipGetLastError());

@@ -31,7 +31,8 @@ template <typename R> struct KArgs {
     Queue<R> qp;             // photon output queue
     Queue<R> qe;             // charged-particle output queue
     DevStatus *status;
-    uint32_t yield_trips;    // loop trips a particle may take per launch
+    uint32_t yield_trips;    // loop trips a particle may take per launch...
+    uint32_t yield_small;    // ...and in a launch whose input holds fewer than drain_min
     uint32_t drain_lanes;    // once the input is used up, a wave with at most
                              // this many live lanes hands its particles on...
     uint32_t drain_trips;    // ...if they have taken this many trips here...
@@ -1017,6 +1018,17 @@ __device__ __forceinline__ int electron_iteration(const KArgs<R> &A, Particle<R>
 }
 
 // ============================================================ kernels =====
+// Lanes of a wavefront that take particles.  A wavefront executes the union
+// of its lanes' paths, so a trip of 64 particles takes two to three times as
+// long as a lone particle's; a launch whose input does not fill its
+// wavefronts spreads the particles over all of them instead (the host sizes
+// the grid of such a launch to SPREAD_WAVES wavefronts per SIMD).
+__device__ __forceinline__ uint32_t lanes_used(uint32_t in_end)
+{
+    const uint32_t waves = gridDim.x * (RNG_LANES / 64);
+    return in_end >= waves * 64u ? 64u : max((in_end + waves - 1u) / waves, 1u);
+}
+
 // Minimum waves per SIMD the register allocation of each transport kernel
 // must allow (the second __launch_bounds__ argument); values above what the
 // kernel needs make the compiler keep fewer values in VGPRs.  Chosen by
@@ -1049,9 +1061,10 @@ __global__ void __launch_bounds__(256, Waves<R>::photon) k_photon(KArgs<R> A)
     PhotonLane<R> s;
     LaneGeo<R> G;
     Scorer<R> sc;
-    bool alive = false, exhausted = false;
     uint32_t nsteps = 0, ncross = 0, trips = 0, here = 0, nyield = 0, longest = 0;
     const uint32_t in_end = min(*A.in_count, A.qin.cap);
+    const uint32_t yield_trips = in_end < A.drain_min ? min(A.yield_trips, A.yield_small) : A.yield_trips;
+    bool alive = false, exhausted = (uint32_t)lane_id() >= lanes_used(in_end);
     for (;;) {
         // free lanes take new particles together (one counter atomic and one
         // round of queue loads for all of them), once enough are free or
@@ -1103,7 +1116,7 @@ __global__ void __launch_bounds__(256, Waves<R>::photon) k_photon(KArgs<R> A)
             if (alive && trips > MAX_ITERS) {           // watchdog: no particle runs forever
                 atomicAdd(&A.status->killed, 1u);
                 alive = false;
-            } else if (alive && s.split == 0u && (here >= A.yield_trips || (drain && here >= A.drain_trips))) {
+            } else if (alive && s.split == 0u && (here >= yield_trips || (drain && here >= A.drain_trips))) {
                 sc.flush(G);
                 yield_push<R>(A.qp, p, s, trips, A.status);
                 nyield++;
@@ -1134,9 +1147,10 @@ __global__ void __launch_bounds__(256, Waves<R>::electron) k_electron(KArgs<R> A
     ElectronLane<R> s;
     LaneGeo<R> G;
     Scorer<R> sc;
-    bool alive = false, exhausted = false;
     uint32_t nsteps = 0, ncross = 0, trips = 0, here = 0, nyield = 0, longest = 0;
     const uint32_t in_end = min(*A.in_count, A.qin.cap);
+    const uint32_t yield_trips = in_end < A.drain_min ? min(A.yield_trips, A.yield_small) : A.yield_trips;
+    bool alive = false, exhausted = (uint32_t)lane_id() >= lanes_used(in_end);
     for (;;) {
         // free lanes take new particles together (one counter atomic and one
         // round of queue loads for all of them), once enough are free or
@@ -1174,7 +1188,7 @@ __global__ void __launch_bounds__(256, Waves<R>::electron) k_electron(KArgs<R> A
             if (r != E_DONE && trips > MAX_ITERS) {     // watchdog: no particle runs forever
                 atomicAdd(&A.status->killed, 1u);
                 r = E_DONE;
-            } else if (r != E_DONE && (here >= A.yield_trips || (drain && here >= A.drain_trips))) {
+            } else if (r != E_DONE && (here >= yield_trips || (drain && here >= A.drain_trips))) {
                 sc.flush(G);
                 yield_push<R>(A.qe, p, s, trips, A.status);
                 nyield++;
