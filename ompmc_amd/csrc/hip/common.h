@@ -285,7 +285,8 @@ template <typename R> struct MsAlias {
 struct MediumScalars {
     double ge0, ge1, eke0, eke1, blcc, xcc, esig_e, psig_e;
     double te, thmoll, ap, delcm, zbrang, bpar0, bpar1, pad;
-    int mono_e, mono_p, meke, pad2;
+    int mono_e, mono_p, meke;
+    int nregular;            // leading electron bins in which zero_ustep's shortcut holds
     double dl1[8], dl2[8], dl3[8], dl4[8], dl5[8], dl6[8];
 };
 
@@ -324,14 +325,67 @@ template <typename R> struct Woodcock {
     int pad;
 };
 
+template <typename R> struct Side2 { R lo, hi; };        // lower and upper bound of a voxel on one axis
+
 template <typename R> struct DevPhantom {
     int isize, jsize, ksize, nreg;
     const double *xb, *yb, *zb;
+    // lower and upper bound of every voxel of each axis, rounded to R: x
+    // voxels, then y, then z.  One load gives both sides of a voxel.
+    const Side2<R> *sides;
     const uint8_t *med;      // [nreg] medium index, 0xff = vacuum / outside
     const R *rhof;           // [nreg]
     double ecut[MAXMED + 1]; // [imed + 1]; entry 0 is vacuum / outside
     double pcut[MAXMED + 1];
     Woodcock<R> wc;
+};
+
+// The medium scalars a charged particle's step reads, copied to LDS at kernel
+// start (values in R where every use converts them): read from the table
+// record in memory they were a chain of dependent loads in every step.
+template <typename R> struct MedRec {
+    double eke0, eke1, te;
+    R keke0, keke1, blcc, xcc, sig_e, sig_p;
+    int mono;                // bit 0 electrons, bit 1 positrons
+    int nregular;
+
+    __device__ __forceinline__ void stage(const MediumScalars &m)
+    {
+        eke0 = m.eke0; eke1 = m.eke1; te = m.te;
+        keke0 = (R)m.eke0; keke1 = (R)m.eke1; blcc = (R)m.blcc; xcc = (R)m.xcc;
+        sig_e = (R)m.esig_e; sig_p = (R)m.psig_e;
+        mono = (m.mono_e ? 1 : 0) | (m.mono_p ? 2 : 0);
+        nregular = m.nregular;
+    }
+};
+
+// The part of a phantom record a transport kernel's lanes read, copied to
+// LDS at kernel start (cut-offs in R, as every use converts them).
+template <typename R> struct GeoRec {
+    int isize, jsize, ksize, nreg;
+    const Side2<R> *sides;
+    const uint8_t *med;
+    const R *rhof;
+    R ecut[MAXMED + 1];      // [imed + 1]; entry 0 is vacuum / outside
+
+    __device__ __forceinline__ void stage(const DevPhantom<R> &p)
+    {
+        isize = p.isize; jsize = p.jsize; ksize = p.ksize; nreg = p.nreg;
+        sides = p.sides; med = p.med; rhof = p.rhof;
+        for (int m = 0; m <= MAXMED; ++m) ecut[m] = (R)p.ecut[m];
+    }
+};
+
+template <typename R> struct PhotonGeoRec : GeoRec<R> {
+    R pcut[MAXMED + 1];
+    Woodcock<R> wc;
+
+    __device__ __forceinline__ void stage(const DevPhantom<R> &p)
+    {
+        GeoRec<R>::stage(p);
+        for (int m = 0; m <= MAXMED; ++m) pcut[m] = (R)p.pcut[m];
+        wc = p.wc;
+    }
 };
 
 // One source job (a dosxyz field, one beamlet, one serving request).
@@ -369,7 +423,7 @@ struct SourceSeg {
 // the middle of its transport (a yield) also carries the lane's state, so
 // the next launch resumes it exactly where it stopped.
 //
-// One allocation per queue: QR_N arrays of R (e x y z u v w wt, then the six
+// One allocation per queue: QR_N arrays of R (e x y z u v w wt, then the five
 // real-valued resume variables), then QU_N arrays of uint32 (ir, meta =
 // job << 3 | resume << 2 | (iq + 1), history index within the job, Philox
 // key and counter, packed integer resume variables, loop trips taken so
@@ -378,7 +432,7 @@ struct SourceSeg {
 // registers; with one pointer per array they took 135 of them and the
 // compiler spilled pointers into vector-register lanes, reading them back
 // before every table or queue access.
-enum { QR_E, QR_X, QR_Y, QR_Z, QR_U, QR_V, QR_W, QR_WT, QR_ST, QR_N = QR_ST + 6 };
+enum { QR_E, QR_X, QR_Y, QR_Z, QR_U, QR_V, QR_W, QR_WT, QR_ST, QR_N = QR_ST + 5 };
 enum { QU_IR, QU_META, QU_HIST, QU_K0, QU_K1, QU_CTR, QU_SFLAGS, QU_TRIPS, QU_N };
 
 template <typename R> struct Queue {

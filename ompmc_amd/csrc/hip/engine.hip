@@ -145,7 +145,7 @@ struct PhantomSlot {
     bool used = false;
     int nreg = 0;
     int isize = 0, jsize = 0, ksize = 0;
-    DevBuf xb, yb, zb, med, rhof, rho;
+    DevBuf xb, yb, zb, sides, med, rhof, rho;
     // delta tracking: largest relative density of each medium (-1 = absent)
     // and the grid, if uniform
     double rho_max[MAXMED];
@@ -529,6 +529,26 @@ template <typename R> static int upload_tables(omc_dev_ctx *c, const omc_tables 
                 d.range = t->range_ep[(size_t)q * nmed * MXEKE + s];
                 d.earr = t->e_array[s];
             }
+    // leading bins of each medium in which a ustep iteration of length 0 is
+    // decided by the energy alone (zero_ustep): tmxs not negative, scattering
+    // power, its correction and stopping power positive at both edges of the
+    // bin, half a bin beyond included (the tables are linear within a bin)
+    for (int m = 0; m < nmed; ++m) {
+        MediumScalars &M = S.med[m];
+        int n = 0;
+        const bool scal = M.eke1 > 0.0 && M.blcc > 0.0 && M.xcc > 0.0;
+        for (bool ok = scal; ok && n < MXEKE; n += ok) {
+            const double edge[2] = { (n + 0.5 - M.eke0) / M.eke1, (n + 2.5 - M.eke0) / M.eke1 };
+            for (int q = 0; q < 2; ++q) {
+                const ElecBin<R> &b = el[((size_t)m * 2 + q) * MXEKE + n];
+                const ElecCsda &d = cs[((size_t)m * 2 + q) * MXEKE + n];
+                for (double x : edge)
+                    ok = ok && x * b.tmxs1 + b.tmxs0 >= 0.0 && x * b.eta1 + b.eta0 > 0.0 &&
+                         x * b.blc1 + b.blc0 > 0.0 && x * d.dedx1 + d.dedx0 > 0.0;
+            }
+        }
+        M.nregular = n;
+    }
     std::vector<R> spin((size_t)nmed * OMC_SPIN_PER_MED);
     for (size_t i = 0; i < spin.size(); ++i) spin[i] = (R)t->spin_rej[i];
     std::vector<MsAlias<R>> ms(OMC_MS_SIZE);
@@ -671,12 +691,17 @@ template <typename R> static int upload_phantom(omc_dev_ctx *c, const omc_phanto
     P.xb.bytes = sizeof(double) * (ph->isize + 1);
     P.yb.bytes = sizeof(double) * (ph->jsize + 1);
     P.zb.bytes = sizeof(double) * (ph->ksize + 1);
+    std::vector<Side2<R>> sides;
+    for (const auto &ax : { std::make_pair(ph->xbounds, ph->isize), std::make_pair(ph->ybounds, ph->jsize),
+                            std::make_pair(ph->zbounds, ph->ksize) })
+        for (int i = 0; i < ax.second; ++i) sides.push_back({ (R)ax.first[i], (R)ax.first[i + 1] });
+    P.sides.bytes = sizeof(Side2<R>) * sides.size();
     P.med.bytes = nreg;
     P.rhof.bytes = sizeof(R) * (size_t)nreg;
     P.rho.bytes = sizeof(double) * (size_t)nvox;
-    DevBuf *bufs[] = { &P.xb, &P.yb, &P.zb, &P.med, &P.rhof, &P.rho };
-    const void *src[] = { ph->xbounds, ph->ybounds, ph->zbounds, med.data(), rhof.data(), ph->rho };
-    for (int b = 0; b < 6; ++b) {
+    DevBuf *bufs[] = { &P.xb, &P.yb, &P.zb, &P.sides, &P.med, &P.rhof, &P.rho };
+    const void *src[] = { ph->xbounds, ph->ybounds, ph->zbounds, sides.data(), med.data(), rhof.data(), ph->rho };
+    for (int b = 0; b < 7; ++b) {
         OMC_TRY_DEV(dalloc(c, &bufs[b]->p, bufs[b]->bytes));
         HIPCHK(hipMemcpy(bufs[b]->p, src[b], bufs[b]->bytes, hipMemcpyHostToDevice));
     }
@@ -684,6 +709,7 @@ template <typename R> static int upload_phantom(omc_dev_ctx *c, const omc_phanto
     memset(&d, 0, sizeof d);
     d.isize = ph->isize; d.jsize = ph->jsize; d.ksize = ph->ksize; d.nreg = nreg;
     d.xb = (const double *)P.xb.p; d.yb = (const double *)P.yb.p; d.zb = (const double *)P.zb.p;
+    d.sides = (const Side2<R> *)P.sides.p;
     d.med = (const uint8_t *)P.med.p; d.rhof = (const R *)P.rhof.p;
     for (int m = 0; m <= MAXMED; ++m) { d.ecut[m] = ecut[m]; d.pcut[m] = pcut[m]; }
     HIPCHK(hipMemcpy((char *)c->d_phantoms + slot * sizeof(DevPhantom<R>), &d, sizeof d, hipMemcpyHostToDevice));
@@ -1504,7 +1530,7 @@ int omc_dev_destroy(omc_dev_ctx *c)
                      c->d_jobs, c->d_phantoms, c->fin_sums };
     for (void *p : ptrs) if (p) (void)hipFree(p);
     for (auto &P : c->ph) {
-        DevBuf *bufs[] = { &P.xb, &P.yb, &P.zb, &P.med, &P.rhof, &P.rho, &P.wc };
+        DevBuf *bufs[] = { &P.xb, &P.yb, &P.zb, &P.sides, &P.med, &P.rhof, &P.rho, &P.wc };
         for (auto *b : bufs) if (b->p) (void)hipFree(b->p);
     }
     for (auto &kv : c->tickets) {
@@ -1549,7 +1575,7 @@ int omc_dev_release_phantom(omc_dev_ctx *c, int id)
     for (auto *w : c->waiting)
         if (w->phantom == id) return fail(OMC_EARG, "phantom %d is in use", id);
     PhantomSlot &P = c->ph[id];
-    DevBuf *bufs[] = { &P.xb, &P.yb, &P.zb, &P.med, &P.rhof, &P.rho, &P.wc };
+    DevBuf *bufs[] = { &P.xb, &P.yb, &P.zb, &P.sides, &P.med, &P.rhof, &P.rho, &P.wc };
     for (auto *b : bufs) { if (b->p) dfree(c, b->p, b->bytes); b->p = nullptr; b->bytes = 0; }
     P.used = false;
     return OMC_OK;

@@ -84,61 +84,84 @@ __device__ __forceinline__ void voxel_of(int irl, int imax, int ijmax, int &irx,
     iry = small_div(rem, imax);
     irx = rem - iry * imax;
 }
-// howfar (omc_dosxyz.c:187-297) for a particle inside region irl > 0.  The
-// boundary each axis heads for is loaded up front (the three loads are in
-// flight together; an axis with zero direction cosine loads one it does not
-// use, always inside the array), then the axes are tested in the
-// reference's order z, x, y.
+// Voxel indices a lane keeps beside its particle's region (valid while the
+// region is not 0): decomposing the region at every use took two divisions,
+// some 50 instructions.
+struct Vox { int x, y, z; };
+
 template <typename R, typename Geo>
-__device__ __forceinline__ void howfar(const Geo &g, int irl, R x, R y, R z, R u, R v, R w,
-                                       int &irnew, R &ustep)
+__device__ __forceinline__ void find_voxel(const Geo &g, int irl, Vox &v)
 {
-    int ijmax = g.isize * g.jsize, imax = g.isize;
-    int irx, iry, irz;
-    voxel_of(irl, imax, ijmax, irx, iry, irz);
-    const R bz = (R)glob(g.zb)[irz + (w > (R)0 ? 1 : 0)];
-    const R bx = (R)glob(g.xb)[irx + (u > (R)0 ? 1 : 0)];
-    const R by = (R)glob(g.yb)[iry + (v > (R)0 ? 1 : 0)];
+    v.x = v.y = v.z = 0;
+    if (irl > 0) voxel_of(irl, g.isize, g.isize * g.jsize, v.x, v.y, v.z);
+}
+
+// The six sides of a voxel.
+template <typename R> struct Sides { R xl, xh, yl, yh, zl, zh; };
+
+template <typename R, typename Geo> __device__ __forceinline__ Sides<R> load_sides(const Geo &g, const Vox &v)
+{
+    const gmem<const Side2<R>> *s = glob(g.sides);
+    const gmem<const Side2<R>> *sx = s + v.x, *sy = s + (g.isize + v.y), *sz = s + (g.isize + g.jsize + v.z);
+    Sides<R> b;
+    b.xl = sx->lo; b.xh = sx->hi;
+    b.yl = sy->lo; b.yh = sy->hi;
+    b.zl = sz->lo; b.zh = sz->hi;
+    return b;
+}
+
+// Which side of its voxel a step crosses: 0 none, +-1 x, +-2 y, +-3 z.  The
+// voxel next to it, or region 0 where the grid ends.
+template <typename Geo> __device__ __forceinline__ void cross_side(const Geo &g, int side, int &ir, Vox &v)
+{
+    const int d = side > 0 ? 1 : -1, axis = side > 0 ? side : -side;
+    const int dx = axis == 1 ? d : 0, dy = axis == 2 ? d : 0, dz = axis == 3 ? d : 0;
+    v.x += dx; v.y += dy; v.z += dz;
+    const bool in = (unsigned)v.x < (unsigned)g.isize && (unsigned)v.y < (unsigned)g.jsize &&
+                    (unsigned)v.z < (unsigned)g.ksize;
+    ir = in ? ir + dx + g.isize * (dy + g.jsize * dz) : 0;
+}
+
+// howfar (omc_dosxyz.c:187-297) for a particle inside a voxel whose sides
+// ahead of it (in the direction of flight, each axis) are ax, ay, az: lowers
+// ustep to the nearest one, axes in the reference's order z, x, y, and names
+// it (0: the step ends inside).  The reference's two forms of the distance,
+// (bound - x)/u and -(x - bound)/u, are the same number.
+template <typename R>
+__device__ __forceinline__ void howfar(R ax, R ay, R az, R x, R y, R z, R u, R v, R w, int &side, R &ustep)
+{
     R dist;
-    if (w > (R)0) {
-        dist = (bz - z) / w;
-        if (dist < ustep) { ustep = dist; irnew = (irz != g.ksize - 1) ? irl + ijmax : 0; }
-    } else if (w < (R)0) {
-        dist = -(z - bz) / w;
-        if (dist < ustep) { ustep = dist; irnew = (irz != 0) ? irl - ijmax : 0; }
+    side = 0;
+    if (w != (R)0) {
+        dist = (az - z) / w;
+        if (dist < ustep) { ustep = dist; side = w > (R)0 ? 3 : -3; }
     }
-    if (u > (R)0) {
-        dist = (bx - x) / u;
-        if (dist < ustep) { ustep = dist; irnew = (irx != g.isize - 1) ? irl + 1 : 0; }
-    } else if (u < (R)0) {
-        dist = -(x - bx) / u;
-        if (dist < ustep) { ustep = dist; irnew = (irx != 0) ? irl - 1 : 0; }
+    if (u != (R)0) {
+        dist = (ax - x) / u;
+        if (dist < ustep) { ustep = dist; side = u > (R)0 ? 1 : -1; }
     }
-    if (v > (R)0) {
-        dist = (by - y) / v;
-        if (dist < ustep) { ustep = dist; irnew = (iry != g.jsize - 1) ? irl + imax : 0; }
-    } else if (v < (R)0) {
-        dist = -(y - by) / v;
-        if (dist < ustep) { ustep = dist; irnew = (iry != 0) ? irl - imax : 0; }
+    if (v != (R)0) {
+        dist = (ay - y) / v;
+        if (dist < ustep) { ustep = dist; side = v > (R)0 ? 2 : -2; }
     }
 }
 
-// hownear (omc_dosxyz.c:299-334)
-template <typename R, typename Geo>
-__device__ __forceinline__ R hownear(const Geo &g, int irl, R x, R y, R z)
+template <typename R>
+__device__ __forceinline__ void howfar(const Sides<R> &b, R x, R y, R z, R u, R v, R w, int &side, R &ustep)
 {
-    if (irl == 0) return (R)0;
-    int ijmax = g.isize * g.jsize, imax = g.isize;
-    int irx, iry, irz;
-    voxel_of(irl, imax, ijmax, irx, iry, irz);
-    const gmem<const double> *xb = glob(g.xb), *yb = glob(g.yb), *zb = glob(g.zb);
+    howfar<R>(u > (R)0 ? b.xh : b.xl, v > (R)0 ? b.yh : b.yl, w > (R)0 ? b.zh : b.zl, x, y, z, u, v, w, side, ustep);
+}
+
+// hownear (omc_dosxyz.c:299-334)
+template <typename R> __device__ __forceinline__ R hownear(const Sides<R> &b, R x, R y, R z)
+{
     R t = (R)1.0E10;
-    t = m_fmin(t, (R)xb[irx + 1] - x);
-    t = m_fmin(t, x - (R)xb[irx]);
-    t = m_fmin(t, (R)yb[iry + 1] - y);
-    t = m_fmin(t, y - (R)yb[iry]);
-    t = m_fmin(t, (R)zb[irz + 1] - z);
-    t = m_fmin(t, z - (R)zb[irz]);
+    t = m_fmin(t, b.xh - x);
+    t = m_fmin(t, x - b.xl);
+    t = m_fmin(t, b.yh - y);
+    t = m_fmin(t, y - b.yl);
+    t = m_fmin(t, b.zh - z);
+    t = m_fmin(t, z - b.zl);
     return t;
 }
 

@@ -243,12 +243,12 @@ __device__ void mscat(const DevTables<R> &T, Rng &rng, int imed, int qel, bool &
 // msdist (ompmc.c:3787-3976): PRESTA-II substeps; moves p to the step end
 // position and direction, returns the straight-line distance.
 template <typename R>
-__device__ __forceinline__ R msdist(const DevTables<R> &T, Particle<R> &p, int imed, R rhof, R de, R tustep, R eke)
+__device__ __forceinline__ R msdist(const DevTables<R> &T, const MedRec<R> &M, Particle<R> &p, int imed, R rhof,
+                                    R de, R tustep, R eke)
 {
-    const MediumScalars &M = T.small->med[imed];
     const int qel = (1 + p.iq) / 2;
     const R rm = (R)RM;
-    R blccc = (R)M.blcc, xcccc = (R)M.xcc;
+    R blccc = M.blcc, xcccc = M.xcc;
     R e = eke - (R)0.5 * de;
     R tau = e / rm;
     R tau2 = sq(tau);

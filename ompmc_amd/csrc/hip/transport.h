@@ -46,12 +46,12 @@ template <typename R> struct KArgs {
 // Per-lane geometry / scoring context for the particle the lane holds.  The
 // phantom records are copied to LDS at kernel start, so a lane keeps one
 // pointer to its record instead of the record's fields.
-template <typename R> struct LaneGeo {
-    const DevPhantom<R> *g;  // LDS copy of the particle's phantom record
+template <typename R, typename Rec> struct LaneGeo {
+    const Rec *g;            // LDS copy of the particle's phantom record
     gmem<double> *tally;     // job tally row of this history's batch
     gmem<double> *ledger;    // job ledger entry of this history (or null)
 
-    __device__ __forceinline__ void bind(const KArgs<R> &A, const DevPhantom<R> *lds, const Particle<R> &p)
+    __device__ __forceinline__ void bind(const KArgs<R> &A, const Rec *lds, const Particle<R> &p)
     {
         const DevJob &J = A.jobs[p.job];
         g = &lds[J.phantom];
@@ -63,16 +63,15 @@ template <typename R> struct LaneGeo {
     __device__ __forceinline__ R rho(int ir) const { return glob(g->rhof)[ir]; }
 };
 
-// Copies the resident phantom records to LDS (all threads of the block).
-template <typename R>
-__device__ __forceinline__ void stage_phantoms(const DevPhantom<R> *src, DevPhantom<R> *lds)
+template <typename R> using PhotonGeo = LaneGeo<R, PhotonGeoRec<R>>;
+template <typename R> using ElectronGeo = LaneGeo<R, GeoRec<R>>;
+
+// Copies the resident phantom records to LDS (all threads of the block; the
+// caller synchronises it).
+template <typename R, typename Rec>
+__device__ __forceinline__ void stage_phantoms(const DevPhantom<R> *src, Rec *lds)
 {
-    constexpr int words = (int)(sizeof(DevPhantom<R>) * MAX_PHANTOMS / 4);
-    static_assert(sizeof(DevPhantom<R>) % 4 == 0, "phantom record must be word sized");
-    const uint32_t *s = reinterpret_cast<const uint32_t *>(src);
-    uint32_t *d = reinterpret_cast<uint32_t *>(lds);
-    for (int i = threadIdx.x; i < words; i += blockDim.x) d[i] = s[i];
-    __syncthreads();
+    if (threadIdx.x < MAX_PHANTOMS) lds[threadIdx.x].stage(src[threadIdx.x]);
 }
 
 // Deposit accumulator: consecutive deposits into the same region are summed
@@ -81,7 +80,7 @@ template <typename R> struct Scorer {
     int ir = -1;
     double acc = 0.0;
     uint32_t ndep = 0;
-    __device__ __forceinline__ void flush(const LaneGeo<R> &G)
+    template <typename Geo> __device__ __forceinline__ void flush(const Geo &G)
     {
         if (ir >= 0) {
             atomicAdd((double *)(G.tally + ir), acc);
@@ -95,7 +94,7 @@ template <typename R> struct Scorer {
         acc = 0.0;
     }
     // ausgab (omc_dosxyz.c:683-694): wt * edep into region ir
-    __device__ __forceinline__ void add(const LaneGeo<R> &G, int region, double e)
+    template <typename Geo> __device__ __forceinline__ void add(const Geo &G, int region, double e)
     {
         ndep++;
         if (region != ir) {
@@ -165,7 +164,7 @@ template <typename R> struct PhotonLane {
     R eta, dpmfp_old;
 
     // After the particle's voxel or energy was set from outside the step.
-    __device__ __forceinline__ void attach(const LaneGeo<R> &G, const Particle<R> &p)
+    __device__ __forceinline__ void attach(const PhotonGeo<R> &G, const Particle<R> &p)
     {
         rhof = G.rho(p.ir);
         cmed = -2;
@@ -206,7 +205,7 @@ __device__ __forceinline__ void detach_stream(const Particle<R> &p, Particle<R> 
 //
 // Next sub-photon, or false when all are done (ompmc.c:1924-1935).
 template <typename R>
-__device__ __forceinline__ bool next_split(Particle<R> &p, PhotonLane<R> &s, LaneGeo<R> &G)
+__device__ __forceinline__ bool next_split(Particle<R> &p, PhotonLane<R> &s, PhotonGeo<R> &G)
 {
     const uint32_t nsplit = s.split & 1023u, isplit = s.split >> 20;
     if (isplit >= nsplit) return false;
@@ -224,7 +223,7 @@ __device__ __forceinline__ bool next_split(Particle<R> &p, PhotonLane<R> &s, Lan
 // Interaction of a sub-photon (ompmc.c:2022-2093), then the next one.
 template <typename R>
 __device__ __forceinline__ bool split_interaction(const KArgs<R> &A, Particle<R> &p, PhotonLane<R> &s,
-                                                  LaneGeo<R> &G)
+                                                  PhotonGeo<R> &G)
 {
     const DevTables<R> &T = A.T;
     const uint32_t nsplit = s.split & 1023u;
@@ -268,7 +267,7 @@ __device__ __forceinline__ bool split_interaction(const KArgs<R> &A, Particle<R>
         }
     } else {
         count_event_global(A.status, EV_PHOTO);
-        photo<R>(q, (R)G.g->ecut[imed + 1]);
+        photo<R>(q, G.g->ecut[imed + 1]);
         p.rng = q.rng;
         detach_stream<R>(p, q);
         push<R>(A.qe, q, A.status);
@@ -288,7 +287,7 @@ __device__ __forceinline__ bool split_interaction(const KArgs<R> &A, Particle<R>
 // Returns true while the photon is still owned by the lane.  Electrons it
 // sets in motion are pushed to A.qe.
 template <typename R>
-__device__ __forceinline__ bool photon_event(const KArgs<R> &A, Particle<R> &p, PhotonLane<R> &s, LaneGeo<R> &G,
+__device__ __forceinline__ bool photon_event(const KArgs<R> &A, Particle<R> &p, PhotonLane<R> &s, PhotonGeo<R> &G,
                                              Scorer<R> &sc)
 {
     const DevTables<R> &T = A.T;
@@ -318,7 +317,7 @@ __device__ __forceinline__ bool photon_event(const KArgs<R> &A, Particle<R> &p, 
                 push<R>(A.qe, b, A.status);
             } else {
                 count_event_global(A.status, EV_PHOTO);
-                photo<R>(p, (R)G.g->ecut[imed + 1]);
+                photo<R>(p, G.g->ecut[imed + 1]);
                 push<R>(A.qe, p, A.status);
                 return false;
             }
@@ -329,7 +328,7 @@ __device__ __forceinline__ bool photon_event(const KArgs<R> &A, Particle<R> &p, 
     s.imed = G.medium(irl);
     s.attach(G, p);
     s.eig = p.e;
-    if (p.e <= (R)G.g->pcut[s.imed + 1] || p.wt == (R)0) {
+    if (p.e <= G.g->pcut[s.imed + 1] || p.wt == (R)0) {
         sc.add(G, irl, (double)p.wt * (double)p.e);
         return false;
     }
@@ -390,7 +389,7 @@ __device__ __forceinline__ void advance(R &x, R &y, R &z, R u, R v, R w, R ustep
 }
 
 template <typename R>
-__device__ __forceinline__ bool photon_step(const KArgs<R> &A, Particle<R> &p, PhotonLane<R> &s, LaneGeo<R> &G,
+__device__ __forceinline__ bool photon_step(const KArgs<R> &A, Particle<R> &p, PhotonLane<R> &s, PhotonGeo<R> &G,
                                             uint32_t &nsteps, uint32_t &ncross)
 {
     const DevTables<R> &T = A.T;
@@ -399,19 +398,40 @@ __device__ __forceinline__ bool photon_step(const KArgs<R> &A, Particle<R> &p, P
     R dk[K], rhok[K];
     int n = 0;
     {
+        const PhotonGeoRec<R> &g = *G.g;
         int irc = p.ir;
+        Vox v;
+        find_voxel<R>(g, irc, v);
         R x = p.x, y = p.y, z = p.z;
+        // the sides ahead on each axis; a crossing replaces only its own
+        R ax = 0, ay = 0, az = 0;
+        const gmem<const Side2<R>> *sides = glob(g.sides);
+        if (irc != 0) {
+            const Sides<R> b = load_sides<R>(g, v);
+            ax = p.u > (R)0 ? b.xh : b.xl;
+            ay = p.v > (R)0 ? b.yh : b.yl;
+            az = p.w > (R)0 ? b.zh : b.zl;
+        }
 #pragma unroll
         for (int k = 0; k < K; ++k) {
             if (irc != 0 && n == k) {
-                int irn = irc;
+                int side;
                 R us = (R)3.0E38;
-                howfar<R>(*G.g, irc, x, y, z, p.u, p.v, p.w, irn, us);
+                howfar<R>(ax, ay, az, x, y, z, p.u, p.v, p.w, side, us);
                 advance<R>(x, y, z, p.u, p.v, p.w, us);
-                irk[k] = irn;
+                cross_side(g, side, irc, v);
+                irk[k] = irc;
                 dk[k] = us;
-                irc = irn;
                 n = k + 1;
+                if (irc != 0 && side != 0) {
+                    const int axis = side > 0 ? side : -side;
+                    const int at = axis == 1 ? v.x : axis == 2 ? g.isize + v.y : g.isize + g.jsize + v.z;
+                    const Side2<R> s2 = { sides[at].lo, sides[at].hi };
+                    const R a = side > 0 ? s2.hi : s2.lo;
+                    if (axis == 1) ax = a;
+                    else if (axis == 2) ay = a;
+                    else az = a;
+                }
             }
         }
 #pragma unroll
@@ -489,11 +509,11 @@ __device__ __forceinline__ bool photon_step(const KArgs<R> &A, Particle<R> &p, P
 #define OMC_WOODCOCK_SITES 8
 #endif
 template <typename R>
-__device__ __forceinline__ bool photon_flight(const KArgs<R> &A, Particle<R> &p, PhotonLane<R> &s, LaneGeo<R> &G,
+__device__ __forceinline__ bool photon_flight(const KArgs<R> &A, Particle<R> &p, PhotonLane<R> &s, PhotonGeo<R> &G,
                                               uint32_t &nsteps, uint32_t &ncross)
 {
     const DevTables<R> &T = A.T;
-    const DevPhantom<R> &g = *G.g;
+    const PhotonGeoRec<R> &g = *G.g;
     const Woodcock<R> &W = g.wc;
     const R mu_max = glob(W.mu)[pwlf_bin(s.gle, (R)W.ge1, (R)W.ge0, MXGE)];
     for (int k = 0; k < OMC_WOODCOCK_SITES; ++k) {
@@ -538,20 +558,23 @@ __device__ __forceinline__ bool photon_flight(const KArgs<R> &A, Particle<R> &p,
 
 // ================================================== electrons/positrons ====
 template <typename R> struct ElectronLane {
-    int phase;               // 0 entry, 1 head of tstep loop, 2 ustep iteration
+    // 0 entry, 1 head of the tstep loop, 2 ustep iteration, 3 head of the
+    // tstep loop with eke, elke and lelke already those of energy and medium
+    int phase;
     int imed, medold, lelke, compute_tstep;
-    R rhof, eke, elke, demfp, sig0, ustep;
+    R rhof, eke, elke, demfp, sig0;
+    Vox vox;                 // not part of the saved state: voxel of the particle's region
 
     __device__ __forceinline__ void save(const Queue<R> &q, uint32_t i) const
     {
         q.st(0)[i] = rhof; q.st(1)[i] = eke; q.st(2)[i] = elke;
-        q.st(3)[i] = demfp; q.st(4)[i] = sig0; q.st(5)[i] = ustep;
+        q.st(3)[i] = demfp; q.st(4)[i] = sig0;
         q.sflags()[i] = pack_lane(phase, compute_tstep, imed, medold, lelke);
     }
     __device__ __forceinline__ void load(const Queue<R> &q, uint32_t i)
     {
         rhof = q.st(0)[i]; eke = q.st(1)[i]; elke = q.st(2)[i];
-        demfp = q.st(3)[i]; sig0 = q.st(4)[i]; ustep = q.st(5)[i];
+        demfp = q.st(3)[i]; sig0 = q.st(4)[i];
         unpack_lane(q.sflags()[i], phase, compute_tstep, imed, medold, lelke);
     }
 };
@@ -593,7 +616,7 @@ __device__ __forceinline__ void push_photon_pair(const KArgs<R> &A, Particle<R> 
 // electron_cutoff: kinetic energy deposited; a positron then annihilates at
 // rest and the lane hands both photons to the photon queue.
 template <typename R>
-__device__ __forceinline__ void electron_cutoff(const KArgs<R> &A, Particle<R> &p, LaneGeo<R> &G,
+__device__ __forceinline__ void electron_cutoff(const KArgs<R> &A, Particle<R> &p, ElectronGeo<R> &G,
                                                 Scorer<R> &sc, R eie)
 {
     R edep = p.e - (R)RM;
@@ -628,7 +651,7 @@ __device__ __forceinline__ int electron_interaction(const KArgs<R> &A, Particle<
         R rfict = urand<R>(p.rng);
         if (rfict >= sigratio) {
             count_event(EV_FICT);
-            s.phase = 1;
+            s.phase = 3;
             return E_ALIVE;
         }
     }
@@ -677,82 +700,56 @@ __device__ __forceinline__ int electron_interaction(const KArgs<R> &A, Particle<
     return E_DONE;
 }
 
+// Moves the particle into the voxel its step crosses to.
+template <typename R>
+__device__ __forceinline__ void enter_voxel(Particle<R> &p, ElectronLane<R> &s, ElectronGeo<R> &G, int side,
+                                            uint32_t &ncross)
+{
+    ncross++;
+    cross_side(*G.g, side, p.ir, s.vox);
+    s.imed = G.medium(p.ir);
+    s.rhof = G.rho(p.ir);
+}
+
 // The ustep iteration that follows a step in matter while the tstep loop
 // goes on (ompmc.c:4780-5345).  total_tstep starts again at 0 in every
 // iteration (ompmc.c:4787), so here tstep = 0 and the step length is
 // min(0, tmxs): the msdist branch cannot be taken, one random number is
 // drawn for the single-scattering test, the particle does not move, and the
-// tstep loop restarts.  Run in the same trip as the step before it; when an
-// unusual table value would make the general iteration behave otherwise,
-// the general iteration runs instead in the next trip.
+// tstep loop restarts.  The number's value decides nothing as long as tmxs
+// >= 0 and the skin depth, the stopping power and so the largest lambda are
+// positive, which the upload checked for the medium's first nregular bins:
+// there the stream just advances, and of the iteration's geometry only the
+// sign of the distance to the voxel's sides (b) is needed.  Run in the same
+// trip as the step before it; in other bins the general iteration runs in
+// the next trip.
 template <typename R>
-__device__ __forceinline__ int zero_ustep(const KArgs<R> &A, Particle<R> &p, ElectronLane<R> &s, LaneGeo<R> &G,
-                                          Scorer<R> &sc, uint32_t &nsteps, uint32_t &ncross)
+__device__ __forceinline__ int zero_ustep(const KArgs<R> &A, const MedRec<R> &M, Particle<R> &p, ElectronLane<R> &s,
+                                          ElectronGeo<R> &G, Scorer<R> &sc, const Sides<R> &b, uint32_t &nsteps,
+                                          uint32_t &ncross)
 {
-    if (s.compute_tstep || !(s.sig0 > (R)0.0) || s.imed == -1) return E_ALIVE;
-    const DevTables<R> &T = A.T;
-    const R rm = (R)RM;
-    const int iq = p.iq;
-    const int qel = (1 + iq) / 2;
-    const R eie = p.e;
-    int irl = p.ir;
-    const int imed = s.imed;
-    const MediumScalars *M = &T.small->med[imed];
-    const R rhof = s.rhof;
-    const R tstep = (R)(0.0 / (double)rhof);
-    const ElecBin<R> &eb = T.el[(imed * 2 + qel) * MXEKE + s.lelke];
-    const ElecCsda &cs = T.csda[(imed * 2 + qel) * MXEKE + s.lelke];
-    R dedx0 = s.elke * (R)cs.dedx1 + (R)cs.dedx0;
-    R dedx = rhof * dedx0;
-    R tmxs = s.elke * eb.tmxs1 + eb.tmxs0;
-    tmxs /= rhof;
-    // the range term of min(tstep, tmxs, range) is >= 0 and cannot lower it
-    R tustep = m_fmin(tstep, tmxs);
-    R tperp = hownear<R>(*G.g, irl, p.x, p.y, p.z);
-    R blccl = rhof * (R)M->blcc;
-    R xccl = rhof * (R)M->xcc;
-    R p2 = s.eke * (s.eke + (R)2.0 * rm);
-    R beta2 = p2 / (p2 + sq(rm));
-    R etap = s.elke * eb.eta1 + eb.eta0;
-    R ms_corr = s.elke * eb.blc1 + eb.blc0;
-    blccl = blccl / etap / ((R)1.0 + (R)0.25 * etap * xccl / blccl / p2) * ms_corr;
-    R ssmfp = beta2 / blccl;
-    R skindepth = (R)3 * ssmfp;
-    if (!(skindepth > (R)0.0)) return E_ALIVE;
-    tustep = m_fmin(tustep, m_fmax(tperp, skindepth));
-    // from here on the general iteration's path is fixed
+    if (s.compute_tstep || !(s.sig0 > (R)0.0) || s.lelke >= M.nregular || !(s.rhof > (R)0.0)) return E_ALIVE;
     nsteps++;
-    R rnno = urand<R>(p.rng);
-    if (rnno < (R)1.0E-30) rnno = (R)1.0E-30;
-    R lambda = (R)(-1.0) * m_log((R)1.0 - rnno);
-    R lambda_max = (R)0.5 * blccl * rm / dedx;
-    lambda_max *= (s.eke / rm + (R)1.0) * (s.eke / rm + (R)1.0) * (s.eke / rm + (R)1.0);
-    if (!(lambda >= (R)0.0 && lambda_max > (R)0.0)) return E_DONE;   // dropped unscored
-    // tuss >= 0 >= tustep: single scattering stays off
-    R ustep = tustep;
-    int irnew = irl;
-    const int irold = irl;
-    if (!(ustep < tperp)) {
+    p.rng.ctr++;
+    s.phase = 3;
+    if (!((R)0.0 < hownear<R>(b, p.x, p.y, p.z))) {
         count_lane_event(EV_HOWFAR_E);
-        howfar<R>(*G.g, irl, p.x, p.y, p.z, p.u, p.v, p.w, irnew, ustep);
+        int side;
+        R ustep = (R)0.0;
+        howfar<R>(b, p.x, p.y, p.z, p.u, p.v, p.w, side, ustep);
+        if (side != 0) {
+            enter_voxel<R>(p, s, G, side, ncross);
+            if (p.e <= G.g->ecut[s.imed + 1]) { electron_cutoff<R>(A, p, G, sc, p.e); return E_DONE; }
+            s.phase = 1;
+        }
     }
-    if (ustep < (R)0) ustep = (R)0.0;
-    s.ustep = ustep;
-    if (irnew != irold) {
-        ncross++;
-        p.ir = irnew;
-        irl = irnew;
-        s.imed = G.medium(irl);
-        s.rhof = G.rho(irl);
-    }
-    if (eie <= (R)G.g->ecut[s.imed + 1]) { electron_cutoff<R>(A, p, G, sc, eie); return E_DONE; }
-    s.phase = 1;
     return E_ALIVE;
 }
 
 template <typename R>
-__device__ __forceinline__ int electron_iteration(const KArgs<R> &A, Particle<R> &p, ElectronLane<R> &s, LaneGeo<R> &G,
-                                  Scorer<R> &sc, uint32_t &nsteps, uint32_t &ncross)
+__device__ __forceinline__ int electron_iteration(const KArgs<R> &A, const MedRec<R> *media, Particle<R> &p,
+                                                  ElectronLane<R> &s, ElectronGeo<R> &G, Scorer<R> &sc,
+                                                  uint32_t &nsteps, uint32_t &ncross)
 {
     const DevTables<R> &T = A.T;
     const R rm = (R)RM;
@@ -765,27 +762,29 @@ __device__ __forceinline__ int electron_iteration(const KArgs<R> &A, Particle<R>
         s.imed = G.medium(irl);
         s.rhof = G.rho(irl);
         s.medold = s.imed;
-        if (eie <= (R)G.g->ecut[s.imed + 1]) { electron_cutoff<R>(A, p, G, sc, eie); return E_DONE; }
+        if (eie <= G.g->ecut[s.imed + 1]) { electron_cutoff<R>(A, p, G, sc, eie); return E_DONE; }
         s.phase = 1;
     }
-    const MediumScalars *M = s.imed >= 0 ? &T.small->med[s.imed] : nullptr;
-    if (s.phase == 1) {
+    const MedRec<R> &M = media[max(s.imed, 0)];
+    if (s.phase != 2) {
         s.compute_tstep = 1;
         s.eke = eie - rm;
         if (s.imed != -1) {
             R rnno = urand<R>(p.rng);
             if (rnno == (R)0.0) rnno = (R)1.0E-30;
             s.demfp = m_fmax(-m_log(rnno), (R)EPSEMFP);
-            s.elke = m_log(s.eke);
-            s.lelke = pwlf_bin(s.elke, M->eke1, M->eke0, MXEKE);
-            if (qel == 0 ? M->mono_e : M->mono_p) {
+            if (s.phase == 1) {
+                s.elke = m_log(s.eke);
+                s.lelke = pwlf_bin(s.elke, M.keke1, M.keke0, MXEKE);
+            }
+            if (M.mono & (1 << qel)) {
                 const ElecBin<R> &eb = T.el[(s.imed * 2 + qel) * MXEKE + s.lelke];
                 const ElecCsda &cs = T.csda[(s.imed * 2 + qel) * MXEKE + s.lelke];
                 s.sig0 = s.elke * eb.sig1 + eb.sig0;
                 R dedx0 = s.elke * (R)cs.dedx1 + (R)cs.dedx0;
                 s.sig0 /= dedx0;
             } else {
-                s.sig0 = (R)(qel == 0 ? M->esig_e : M->psig_e);
+                s.sig0 = qel == 0 ? M.sig_e : M.sig_p;
             }
         }
         s.phase = 2;
@@ -793,8 +792,10 @@ __device__ __forceinline__ int electron_iteration(const KArgs<R> &A, Particle<R>
 
     // ---- one ustep iteration ----
     nsteps++;
-    int irl = p.ir;
-    int imed = s.imed;
+    const int irl = p.ir;
+    const int imed = s.imed;
+    Sides<R> b = {};
+    if (irl != 0) b = load_sides<R>(*G.g, s.vox);
     bool call_howfar, do_single = false, called_msdist = false;
     R tstep, tustep, range = 0, tvstep = 0, de = 0, tperp = 0;
     double total_tstep = 0.0;             // fresh every iteration (ompmc.c:4787)
@@ -808,7 +809,7 @@ __device__ __forceinline__ int electron_iteration(const KArgs<R> &A, Particle<R>
         call_howfar = true;
     } else {
         csb = T.csda + (imed * 2 + qel) * MXEKE;
-        const double eke0 = M->eke0, eke1 = M->eke1;
+        const double eke0 = M.eke0, eke1 = M.eke1;
         const R rhof = s.rhof;          // density of the current voxel, loaded on entering it
         if (s.sig0 <= (R)0.0) {
             tstep = (R)10.0E8;
@@ -856,9 +857,9 @@ __device__ __forceinline__ int electron_iteration(const KArgs<R> &A, Particle<R>
             range = (R)rg;
         }
         tustep = m_fmin(m_fmin(tstep, tmxs), range);
-        tperp = hownear<R>(*G.g, irl, p.x, p.y, p.z);
-        R blccl = rhof * (R)M->blcc;
-        R xccl = rhof * (R)M->xcc;
+        tperp = hownear<R>(b, p.x, p.y, p.z);
+        R blccl = rhof * M.blcc;
+        R xccl = rhof * M.xcc;
         R p2 = s.eke * (s.eke + (R)2.0 * rm);
         R beta2 = p2 / (p2 + sq(rm));
         R etap = s.elke * eb.eta1 + eb.eta0;
@@ -871,14 +872,14 @@ __device__ __forceinline__ int electron_iteration(const KArgs<R> &A, Particle<R>
             call_howfar = false;
             do_single = false;
             called_msdist = true;
-            de = (R)eloss(csb, M->te, eke0, eke1, (double)rhof, (double)tustep, (double)range,
+            de = (R)eloss(csb, M.te, eke0, eke1, (double)rhof, (double)tustep, (double)range,
                           (double)s.eke, (double)s.elke, s.lelke);
             tvstep = tustep;
             // msdist moves a copy; the original position is kept until
             // after ausgab, which scores in the pre-step region
             Particle<R> q = p;
             count_lane_event(EV_MSDIST);
-            ustep = msdist<R>(T, q, imed, rhof, de, tustep, s.eke);
+            ustep = msdist<R>(T, M, q, imed, rhof, de, tustep, s.eke);
             p.rng = q.rng;
             xf = q.x; yf = q.y; zf = q.z; uf = q.u; vf = q.v; wf = q.w;
         } else {
@@ -902,7 +903,7 @@ __device__ __forceinline__ int electron_iteration(const KArgs<R> &A, Particle<R>
         }
     }
 
-    int irold = p.ir, irnew = p.ir;
+    int side = 0;                            // side of the voxel the step crosses
     if (call_howfar) {
         count_lane_event(EV_HOWFAR_E);
         if (irl == 0) {                      // howfar discard (outside)
@@ -916,10 +917,9 @@ __device__ __forceinline__ int electron_iteration(const KArgs<R> &A, Particle<R>
             }
             return E_DONE;
         }
-        howfar<R>(*G.g, irl, p.x, p.y, p.z, p.u, p.v, p.w, irnew, ustep);
+        howfar<R>(b, p.x, p.y, p.z, p.u, p.v, p.w, side, ustep);
     }
     if (ustep < (R)0) ustep = (R)0.0;
-    s.ustep = ustep;
     if (ustep == (R)0.0 || imed == -1) {
         if (ustep != (R)0.0) {
             R vstep = ustep;
@@ -927,14 +927,8 @@ __device__ __forceinline__ int electron_iteration(const KArgs<R> &A, Particle<R>
             p.y += p.v * vstep;
             p.z += p.w * vstep;
         }
-        if (irnew != irold) {
-            ncross++;
-            p.ir = irnew;
-            irl = irnew;
-            s.imed = G.medium(irl);
-            s.rhof = G.rho(irl);
-        }
-        if (eie <= (R)G.g->ecut[s.imed + 1]) { electron_cutoff<R>(A, p, G, sc, eie); return E_DONE; }
+        if (side != 0) enter_voxel<R>(p, s, G, side, ncross);
+        if (eie <= G.g->ecut[s.imed + 1]) { electron_cutoff<R>(A, p, G, sc, eie); return E_DONE; }
         // leave the ustep loop; the tstep loop restarts unless a step through
         // vacuum brought the particle back into the medium it last lost energy
         // in, where the reference goes on to the fictitious-sigma test
@@ -950,12 +944,12 @@ __device__ __forceinline__ int electron_iteration(const KArgs<R> &A, Particle<R>
     if (call_howfar) {
         tvstep = vstep;
         if (tvstep != tustep) do_single = false;
-        de = (R)eloss(csb, M->te, M->eke0, M->eke1, (double)rhof, (double)tvstep, (double)range,
+        de = (R)eloss(csb, M.te, M.eke0, M.eke1, (double)rhof, (double)tvstep, (double)range,
                       (double)s.eke, (double)s.elke, s.lelke);
     } else {
         tvstep = tustep;
         if (!called_msdist)
-            de = (R)eloss(csb, M->te, M->eke0, M->eke1, (double)rhof, (double)tvstep, (double)range,
+            de = (R)eloss(csb, M.te, M.eke0, M.eke1, (double)rhof, (double)tvstep, (double)range,
                           (double)s.eke, (double)s.elke, s.lelke);
     }
     R edep = de;
@@ -963,12 +957,12 @@ __device__ __forceinline__ int electron_iteration(const KArgs<R> &A, Particle<R>
     if (!called_msdist) {
         R sinthe, costhe;
         if (do_single) {
-            R ekems = m_fmax(ekef, (R)G.g->ecut[imed + 1] - rm);
+            R ekems = m_fmax(ekef, G.g->ecut[imed + 1] - rm);
             R p2 = ekems * (ekems + (R)2.0 * rm);
             R beta2 = p2 / (p2 + sq(rm));
-            R chia2 = (R)M->xcc / ((R)4.0 * (R)M->blcc * p2);
+            R chia2 = M.xcc / ((R)4.0 * M.blcc * p2);
             R elkems = m_log(ekems);
-            int lelkems = pwlf_bin(elkems, M->eke1, M->eke0, MXEKE);
+            int lelkems = pwlf_bin(elkems, M.keke1, M.keke0, MXEKE);
             const ElecBin<R> &ebs = T.el[(imed * 2 + qel) * MXEKE + lelkems];
             R etap = elkems * ebs.eta1 + ebs.eta0;
             chia2 *= etap;
@@ -990,29 +984,25 @@ __device__ __forceinline__ int electron_iteration(const KArgs<R> &A, Particle<R>
     sc.add(G, p.ir, (double)p.wt * (double)edep);
     p.x = xf; p.y = yf; p.z = zf;
     p.u = uf; p.v = vf; p.w = wf;
-    irold = p.ir;
     eie -= edep;
     p.e = eie;
-    if (irnew == irl && eie <= (R)G.g->ecut[imed + 1]) { electron_cutoff<R>(A, p, G, sc, eie); return E_DONE; }
+    if (side == 0 && eie <= G.g->ecut[imed + 1]) { electron_cutoff<R>(A, p, G, sc, eie); return E_DONE; }
     s.medold = imed;
     if (imed != -1) {
         s.eke = eie - rm;
         s.elke = m_log(s.eke);
-        s.lelke = pwlf_bin(s.elke, M->eke1, M->eke0, MXEKE);
+        s.lelke = pwlf_bin(s.elke, M.keke1, M.keke0, MXEKE);
     }
-    if (irnew != irold) {
-        ncross++;
-        p.ir = irnew;
-        irl = irnew;
-        s.imed = G.medium(irl);
-        s.rhof = G.rho(irl);
+    if (side != 0) {
+        enter_voxel<R>(p, s, G, side, ncross);
+        if (p.ir != 0) b = load_sides<R>(*G.g, s.vox);
     }
-    if (eie <= (R)G.g->ecut[s.imed + 1]) { electron_cutoff<R>(A, p, G, sc, eie); return E_DONE; }
+    if (eie <= G.g->ecut[s.imed + 1]) { electron_cutoff<R>(A, p, G, sc, eie); return E_DONE; }
     if (s.imed != s.medold) { s.phase = 1; return E_ALIVE; }
     s.demfp -= de * s.sig0;
     total_tstep -= (double)tvstep * (double)rhof;
     if (total_tstep < 1.0E-9) s.demfp = (R)0.0;
-    if (s.demfp >= (R)EPSEMFP) return zero_ustep<R>(A, p, s, G, sc, nsteps, ncross);
+    if (s.demfp >= (R)EPSEMFP) return zero_ustep<R>(A, M, p, s, G, sc, b, nsteps, ncross);
 
     return electron_interaction<R>(A, p, s);
 }
@@ -1055,11 +1045,12 @@ template <> struct Waves<double> { static constexpr int photon = OMC_WAVES_P64, 
 template <typename R>
 __global__ void __launch_bounds__(256, Waves<R>::photon) k_photon(KArgs<R> A)
 {
-    __shared__ DevPhantom<R> lds_ph[MAX_PHANTOMS];
-    stage_phantoms<R>(A.phantoms, lds_ph);
+    __shared__ PhotonGeoRec<R> lds_ph[MAX_PHANTOMS];
+    stage_phantoms(A.phantoms, lds_ph);
+    __syncthreads();
     Particle<R> p;
     PhotonLane<R> s;
-    LaneGeo<R> G;
+    PhotonGeo<R> G;
     Scorer<R> sc;
     uint32_t nsteps = 0, ncross = 0, trips = 0, here = 0, nyield = 0, longest = 0;
     const uint32_t in_end = min(*A.in_count, A.qin.cap);
@@ -1140,12 +1131,15 @@ __global__ void __launch_bounds__(256, Waves<R>::photon) k_photon(KArgs<R> A)
 template <typename R>
 __global__ void __launch_bounds__(256, Waves<R>::electron) k_electron(KArgs<R> A)
 {
-    __shared__ DevPhantom<R> lds_ph[MAX_PHANTOMS];
+    __shared__ GeoRec<R> lds_ph[MAX_PHANTOMS];
+    __shared__ MedRec<R> media[MAXMED];
     events_begin<true>();
-    stage_phantoms<R>(A.phantoms, lds_ph);
+    stage_phantoms(A.phantoms, lds_ph);
+    if (threadIdx.x >= 64 && threadIdx.x < 64 + MAXMED) media[threadIdx.x - 64].stage(A.T.small->med[threadIdx.x - 64]);
+    __syncthreads();
     Particle<R> p;
     ElectronLane<R> s;
-    LaneGeo<R> G;
+    ElectronGeo<R> G;
     Scorer<R> sc;
     uint32_t nsteps = 0, ncross = 0, trips = 0, here = 0, nyield = 0, longest = 0;
     const uint32_t in_end = min(*A.in_count, A.qin.cap);
@@ -1170,6 +1164,7 @@ __global__ void __launch_bounds__(256, Waves<R>::electron) k_electron(KArgs<R> A
                     trips = 0;
                 }
                 G.bind(A, lds_ph, p);
+                find_voxel<R>(*G.g, p.ir, s.vox);
                 here = 0;
                 alive = true;
             } else {
@@ -1182,7 +1177,7 @@ __global__ void __launch_bounds__(256, Waves<R>::electron) k_electron(KArgs<R> A
             in_end >= A.drain_min && __ballot(exhausted) != 0 && (uint32_t)__popcll(live) <= A.drain_lanes;
         ring_fill(p.rng, alive, live);
         if (alive) {
-            int r = electron_iteration<R>(A, p, s, G, sc, nsteps, ncross);
+            int r = electron_iteration<R>(A, media, p, s, G, sc, nsteps, ncross);
             ++trips;
             ++here;
             if (r != E_DONE && trips > MAX_ITERS) {     // watchdog: no particle runs forever
