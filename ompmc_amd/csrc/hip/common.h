@@ -413,10 +413,11 @@ struct DevJob {
 };
 
 // A run of consecutive histories [first, first + n) of one job, placed at
-// thread offset `off` of a source launch.
+// thread offset `off` of a source launch and at entry `slot` of the queue of
+// its particles' type.
 struct SourceSeg {
     uint64_t first;
-    uint32_t job, n, off, pad;
+    uint32_t job, n, off, slot;
 };
 
 // Structure-of-arrays particle queue.  A particle that gave up its lane in
@@ -544,14 +545,6 @@ template <bool LANES> __device__ __forceinline__ void events_begin()
 // wavefront are serialised by the LDS, which costs little for events that
 // come a few times per history).
 __device__ __forceinline__ void count_event(int k) { atomicAdd(&ev_block[k], 1u); }
-
-// A rare event in every active lane, straight into the launch status: one
-// global atomic per wavefront (kernels that keep no block counters).
-__device__ __forceinline__ void count_event_global(DevStatus *st, int k)
-{
-    const uint64_t m = __ballot(1);
-    if (lane_id() == __ffsll((unsigned long long)m) - 1) atomicAdd(&st->ev[k], (unsigned long long)__popcll(m));
-}
 
 // A frequent event of this thread's lane.
 __device__ __forceinline__ void count_lane_event(int k) { ev_lane[k - EV_NRARE][threadIdx.x] += 1u; }

@@ -94,7 +94,8 @@ constexpr int64_t DEFAULT_CHUNK = 1 << 22;
 constexpr int64_t MAX_SPLIT_INFLIGHT = 16;
 constexpr uint32_t DEFAULT_YIELD_TRIPS = 4096;
 // A launch whose input is below the drain threshold (it cannot fill the
-// device) hands its particles on after this many trips: the photons that its
+// device) but more than four particles to a wavefront hands its particles on
+// after this many trips: the photons that its
 // charged particles have made by then are followed while its longest tracks
 // go on, instead of after them, and the tracks left are spread over the
 // device again.  A generation costs about 0.2 ms, as much as 40 trips of a
@@ -1051,7 +1052,7 @@ static int pull_segments(omc_dev_ctx *c, int pi, int64_t room, uint32_t &injP, u
         sg.job = (uint32_t)j;
         sg.n = (uint32_t)take;
         sg.off = off;
-        sg.pad = 0;
+        sg.slot = J.w->tmpl.charge == 0 ? P.nP + injP : P.nE + injE;
         off += (uint32_t)take;
         room -= take * weight;
         J.injected += take;
@@ -1092,7 +1093,7 @@ template <typename R> static int launch_generation(omc_dev_ctx *c, int pi)
         HIPCHK(hipMemcpyAsync(P.d_segs, P.h->segs, nseg * sizeof(SourceSeg), hipMemcpyHostToDevice, s));
         HIPCHK(hipEventRecord(P.ev_src0, s));
         Launch<R>::source(c->d_jobs, (const DevPhantom<R> *)c->d_phantoms, P.d_segs, nseg, ntot, qpc, qec,
-                          P.d_status, s);
+                          inP, inE, P.d_status, s);
         HIPCHK(hipEventRecord(P.ev_src1, s));
     }
     // The photon kernel appends the electrons it sets in motion to the

@@ -12,7 +12,8 @@ template <typename R> struct KArgs;
 
 template <typename R> struct Launch {
     static void source(const DevJob *jobs, const DevPhantom<R> *ph, const SourceSeg *segs, int nseg,
-                       uint32_t ntot, const Queue<R> &qp, const Queue<R> &qe, DevStatus *st, hipStream_t s);
+                       uint32_t ntot, const Queue<R> &qp, const Queue<R> &qe, uint32_t endp, uint32_t ende,
+                       DevStatus *st, hipStream_t s);
     static void photon(const KArgs<R> &a, int grid, hipStream_t s);
     static void electron(const KArgs<R> &a, int grid, hipStream_t s);
     static void math_eval(int fn, int64_t n, const double *x, const double *y, double *out, hipStream_t s);

@@ -42,6 +42,12 @@ __device__ __forceinline__ float  m_fabs(float a)  { return fabsf(a); }
 
 template <typename R> __device__ __forceinline__ R sq(R x) { return x * x; }
 
+// A product that is rounded before it is used.  The FP32 build fuses a
+// multiplication with the addition it feeds wherever the compiler finds the
+// two in one block; where that depends on the code around them, this fixes
+// the choice, so that changes around it do not change the histories.
+template <typename R> __device__ __forceinline__ void rounded(R &x) { asm volatile("" : "+v"(x)); }
+
 // pwlfInterval / pwlfEval (ompmc.c:203-211)
 template <typename R, typename T>
 __device__ __forceinline__ int pwlf_idx(R l, T c1, T c0) { return (int)(l * (R)c1 + (R)c0); }
@@ -425,7 +431,9 @@ __device__ void compton(Particle<R> &a, Particle<R> &b)
     } while ((br < bro) || (br > (R)1));
     costhe = (R)1.0 - temp;
     sinthe = m_sqrt(sinthe);
-    R esg = br * eig, ese = eig - esg + rm;
+    R esg = br * eig;
+    rounded(esg);
+    R ese = eig - esg + rm;
     a.e = esg;
     Uphi<R> h;
     uphi21<R>(a, h, costhe, sinthe);

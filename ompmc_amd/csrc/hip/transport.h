@@ -32,7 +32,7 @@ template <typename R> struct KArgs {
     Queue<R> qe;             // charged-particle output queue
     DevStatus *status;
     uint32_t yield_trips;    // loop trips a particle may take per launch...
-    uint32_t yield_small;    // ...and in a launch whose input holds fewer than drain_min
+    uint32_t yield_small;    // ...and in a launch of middling size (trips_per_launch)
     uint32_t drain_lanes;    // once the input is used up, a wave with at most
                              // this many live lanes hands its particles on...
     uint32_t drain_trips;    // ...if they have taken this many trips here...
@@ -233,7 +233,7 @@ __device__ __forceinline__ bool split_interaction(const KArgs<R> &A, Particle<R>
     R rnno = urand<R>(q.rng);
     if (rnno <= (R)1.0 - s.cohfac) {
         if (survivor) {
-            count_event_global(A.status, EV_RAYLEIGH);
+            count_event(EV_RAYLEIGH);
             q.wt *= (R)nsplit;
             rayleigh<R>(T, q, imed, s.eig, s.gle, s.lgle);
             p.rng = q.rng;
@@ -249,14 +249,14 @@ __device__ __forceinline__ bool split_interaction(const KArgs<R> &A, Particle<R>
     R gbr1 = s.gle * br.a1 + br.a0;
     Particle<R> b;
     if (rnno <= gbr1 && s.eig > (R)2.0 * (R)RM) {
-        count_event_global(A.status, EV_PAIR);
+        count_event(EV_PAIR);
         pair<R>(T, q, b, imed);
         p.rng = q.rng;
         detach_stream<R>(p, q);
         push<R>(A.qe, q, A.status);
         push<R>(A.qe, b, A.status);
     } else if (rnno < s.gle * br.b1 + br.b0) {
-        count_event_global(A.status, EV_COMPTON);
+        count_event(EV_COMPTON);
         compton<R>(q, b);
         p.rng = q.rng;
         push<R>(A.qe, b, A.status);
@@ -266,7 +266,7 @@ __device__ __forceinline__ bool split_interaction(const KArgs<R> &A, Particle<R>
             push<R>(A.qp, q, A.status);
         }
     } else {
-        count_event_global(A.status, EV_PHOTO);
+        count_event(EV_PHOTO);
         photo<R>(q, G.g->ecut[imed + 1]);
         p.rng = q.rng;
         detach_stream<R>(p, q);
@@ -274,6 +274,65 @@ __device__ __forceinline__ bool split_interaction(const KArgs<R> &A, Particle<R>
     }
     return next_split<R>(p, s, G);
 }
+
+enum { OUT_MADE = 1u, OUT_SELF = 2u };
+
+// Charged particles a wavefront of the photon kernel has made and not yet
+// queued, in LDS.  All wavefronts of the device reserve queue slots through
+// one counter, which serves an atomic every 11 to 12 ns: reserving for the
+// ten or so lanes of each event was all the photon kernel did with its time
+// (1.15e7 atomics in 118 ms at a sixth of the VALU's issue slots, on 8e7 FP32
+// slab histories).  Up to 64 records go out together instead, with one
+// reservation and coalesced stores: 29.2 -> 16.5 ms per 2e7 histories.
+// Called by the whole wavefront.
+constexpr uint32_t STAGE_ROWS = 64;
+template <typename R> struct StageRows {
+    R r[QR_ST][STAGE_ROWS];
+    uint32_t u[QU_SFLAGS][STAGE_ROWS];
+};
+
+template <typename R> struct Stage {
+    StageRows<R> *rows;
+    uint32_t n = 0;                    // records staged (uniform in the wavefront)
+
+    __device__ __forceinline__ void flush(const Queue<R> &q, DevStatus *st)
+    {
+        if (n == 0) return;
+        const uint32_t lane = (uint32_t)lane_id();
+        uint32_t base = 0;
+        if (lane == 0) base = atomicAdd(q.count, n);
+        base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+        const uint32_t i = base + lane;
+        if (lane < n) {
+            if (i < q.cap) {
+#pragma unroll
+                for (int f = 0; f < QR_ST; ++f) q.r(f)[i] = rows->r[f][lane];
+#pragma unroll
+                for (int f = 0; f < QU_SFLAGS; ++f) q.u(f)[i] = rows->u[f][lane];
+            } else {
+                atomicOr(&st->overflow, 1u);
+            }
+        }
+        n = 0;
+    }
+    __device__ __forceinline__ void push(const Queue<R> &q, bool have, const Particle<R> &p, DevStatus *st)
+    {
+        const uint64_t mask = __ballot(have);
+        const uint32_t add = (uint32_t)__popcll(mask);
+        if (add == 0) return;
+        if (n + add > STAGE_ROWS) flush(q, st);
+        if (have) {
+            const uint32_t k = n + lanes_below(mask);
+            rows->r[QR_E][k] = p.e; rows->r[QR_X][k] = p.x; rows->r[QR_Y][k] = p.y; rows->r[QR_Z][k] = p.z;
+            rows->r[QR_U][k] = p.u; rows->r[QR_V][k] = p.v; rows->r[QR_W][k] = p.w; rows->r[QR_WT][k] = p.wt;
+            rows->u[QU_IR][k] = (uint32_t)p.ir;
+            rows->u[QU_META][k] = (p.job << 3) | (uint32_t)(p.iq + 1);
+            rows->u[QU_HIST][k] = p.hist;
+            rows->u[QU_K0][k] = p.rng.k0; rows->u[QU_K1][k] = p.rng.k1; rows->u[QU_CTR][k] = p.rng.ctr;
+        }
+        n += add;
+    }
+};
 
 // A photon lane alternates transport steps (phase 1) with events: the
 // interaction at the end of a step (phase 2) and the (re-)entry into
@@ -284,11 +343,12 @@ __device__ __forceinline__ bool split_interaction(const KArgs<R> &A, Particle<R>
 
 // Event: the pending interaction (ompmc.c:2026-2068), then the entry into
 // photon() (ompmc.c:1884-1935, nsplit = 1) of the photon that goes on.
-// Returns true while the photon is still owned by the lane.  Electrons it
-// sets in motion are pushed to A.qe.
+// Returns true while the photon is still owned by the lane.  The charged
+// particles it sets in motion are b (out has OUT_MADE) and, where the photon
+// ends in one, p itself (OUT_SELF); the caller queues them.
 template <typename R>
 __device__ __forceinline__ bool photon_event(const KArgs<R> &A, Particle<R> &p, PhotonLane<R> &s, PhotonGeo<R> &G,
-                                             Scorer<R> &sc)
+                                             Scorer<R> &sc, Particle<R> &b, uint32_t &out)
 {
     const DevTables<R> &T = A.T;
     if (s.phase == 2) {
@@ -296,29 +356,27 @@ __device__ __forceinline__ bool photon_event(const KArgs<R> &A, Particle<R> &p, 
         const int imed = s.imed;
         R rnno = urand<R>(p.rng);
         if (rnno <= (R)1.0 - s.cohfac) {
-            count_event_global(A.status, EV_RAYLEIGH);
+            count_event(EV_RAYLEIGH);
             rayleigh<R>(T, p, imed, s.eig, s.gle, s.lgle);
         } else {
             rnno = urand<R>(p.rng);
             R4<R> br = T.ph_br[imed * MXGE + s.lgle];
             R gbr1 = s.gle * br.a1 + br.a0;
-            Particle<R> b;
             if (rnno <= gbr1 && s.eig > (R)2.0 * (R)RM) {
-                count_event_global(A.status, EV_PAIR);
+                count_event(EV_PAIR);
                 pair<R>(T, p, b, imed);
-                push<R>(A.qe, p, A.status);
-                push<R>(A.qe, b, A.status);
+                out = OUT_SELF | OUT_MADE;
                 return false;
             }
             R gbr2 = s.gle * br.b1 + br.b0;
             if (rnno < gbr2) {
-                count_event_global(A.status, EV_COMPTON);
+                count_event(EV_COMPTON);
                 compton<R>(p, b);
-                push<R>(A.qe, b, A.status);
+                out = OUT_MADE;
             } else {
-                count_event_global(A.status, EV_PHOTO);
+                count_event(EV_PHOTO);
                 photo<R>(p, G.g->ecut[imed + 1]);
-                push<R>(A.qe, p, A.status);
+                out = OUT_SELF;
                 return false;
             }
         }
@@ -1019,6 +1077,16 @@ __device__ __forceinline__ uint32_t lanes_used(uint32_t in_end)
     return in_end >= waves * 64u ? 64u : max((in_end + waves - 1u) / waves, 1u);
 }
 
+// Loop trips a particle may take in this launch.  A launch that cannot fill
+// the device (fewer than drain_min particles) hands its tracks on early, so
+// that the photons its charged particles made are followed meanwhile and the
+// tracks left are spread anew; with four or fewer particles to a wavefront
+// there is nothing left to spread, and the launch runs to its end.
+template <typename R> __device__ __forceinline__ uint32_t trips_per_launch(const KArgs<R> &A, uint32_t in_end)
+{
+    return in_end < A.drain_min && lanes_used(in_end) > 4u ? min(A.yield_trips, A.yield_small) : A.yield_trips;
+}
+
 // Minimum waves per SIMD the register allocation of each transport kernel
 // must allow (the second __launch_bounds__ argument); values above what the
 // kernel needs make the compiler keep fewer values in VGPRs.  Chosen by
@@ -1042,10 +1110,52 @@ template <typename R> struct Waves;
 template <> struct Waves<float> { static constexpr int photon = OMC_WAVES_P32, electron = OMC_WAVES_E32; };
 template <> struct Waves<double> { static constexpr int photon = OMC_WAVES_P64, electron = OMC_WAVES_E64; };
 
+// A wavefront's share of the launch's input.  While much of the input is
+// left it takes CHUNK consecutive entries with one atomic and hands them to
+// its lanes as they come free; towards the end only what its lanes need.  All
+// wavefronts of the device add to this one counter, which serves an atomic
+// every 11 to 12 ns.  Photon / charged-particle kernel on 2e7 FP32 slab
+// histories, ms: no chunks 20.9 / 88.3, 16 20.7 / 87.2, 32 18.5 / 85.3, 64
+// 16.2 / 88.4, 128 16.7 / 110, 256 21 / 176: a charged-particle launch reads
+// its longest tracks first, and a large share keeps too many of them in one
+// wavefront.
+constexpr uint32_t FEED_PHOTON = 64, FEED_ELECTRON = 32;
+template <uint32_t CHUNK> struct Feed {
+    uint32_t at = 0, end = 0;          // entries in hand (uniform in the wavefront)
+
+    // An entry for every lane of `mask` (the lanes that want one; all lanes of
+    // the wavefront call it), or an index not below in_end where the input
+    // has ended.
+    __device__ __forceinline__ uint32_t take(uint32_t *fetch, uint32_t in_end, uint64_t mask)
+    {
+        const uint32_t n = (uint32_t)__popcll(mask), rank = lanes_below(mask);
+        const uint32_t have = end - at;
+        uint32_t i = at + rank;
+        if (have >= n) {
+            at += n;
+            return i;
+        }
+        // what is in hand goes to the first lanes, the others start on the next share
+        const uint32_t plenty = gridDim.x * (RNG_LANES / 64) * (2u * CHUNK);
+        const uint32_t want = end < in_end && in_end - end > plenty ? max(CHUNK, n - have) : n - have;
+        uint32_t base = 0;
+        if (lane_id() == 0) base = atomicAdd(fetch, want);
+        base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+        if (rank >= have) i = base + (rank - have);
+        at = base + (n - have);
+        end = base + want;
+        return i;
+    }
+};
+
 template <typename R>
 __global__ void __launch_bounds__(256, Waves<R>::photon) k_photon(KArgs<R> A)
 {
     __shared__ PhotonGeoRec<R> lds_ph[MAX_PHANTOMS];
+    __shared__ StageRows<R> made[RNG_LANES / 64];
+    Stage<R> stage;
+    stage.rows = &made[threadIdx.x >> 6];
+    events_begin<false>();
     stage_phantoms(A.phantoms, lds_ph);
     __syncthreads();
     Particle<R> p;
@@ -1054,7 +1164,8 @@ __global__ void __launch_bounds__(256, Waves<R>::photon) k_photon(KArgs<R> A)
     Scorer<R> sc;
     uint32_t nsteps = 0, ncross = 0, trips = 0, here = 0, nyield = 0, longest = 0;
     const uint32_t in_end = min(*A.in_count, A.qin.cap);
-    const uint32_t yield_trips = in_end < A.drain_min ? min(A.yield_trips, A.yield_small) : A.yield_trips;
+    const uint32_t yield_trips = trips_per_launch(A, in_end);
+    Feed<FEED_PHOTON> feed;
     bool alive = false, exhausted = (uint32_t)lane_id() >= lanes_used(in_end);
     for (;;) {
         // free lanes take new particles together (one counter atomic and one
@@ -1064,9 +1175,9 @@ __global__ void __launch_bounds__(256, Waves<R>::photon) k_photon(KArgs<R> A)
         // only free lanes are active, and a ballot of `alive` there is 0)
         const unsigned long long want = __ballot(!alive && !exhausted);
         const bool none_live = __ballot(alive) == 0;
-        if (!alive && !exhausted && ((uint32_t)__popcll(want) >= A.fetch_min || none_live)) {
-            uint32_t i = wave_reserve(A.fetch, 1);
-            if (i < in_end) {
+        if (want != 0 && ((uint32_t)__popcll(want) >= A.fetch_min || none_live)) {
+            const uint32_t i = feed.take(A.fetch, in_end, want);
+            if (!alive && !exhausted && i < in_end) {
                 if (q_load(A.qin, i, p)) {
                     s.load(A.qin, i);
                     trips = A.qin.trips()[i];
@@ -1079,7 +1190,7 @@ __global__ void __launch_bounds__(256, Waves<R>::photon) k_photon(KArgs<R> A)
                 s.attach(G, p);
                 here = 0;
                 alive = true;
-            } else {
+            } else if (!alive) {
                 exhausted = true;
             }
         }
@@ -1095,9 +1206,11 @@ __global__ void __launch_bounds__(256, Waves<R>::photon) k_photon(KArgs<R> A)
         const uint32_t nev = (uint32_t)__popcll(__ballot(alive && s.phase != 1));
         const bool events = nev * A.event_div >= nlive || nev == nlive;
         ring_fill(p.rng, alive, live);
+        Particle<R> b;
+        uint32_t out = 0u;
         if (alive && (s.phase == 1 || events)) {
             if (s.phase != 1)
-                alive = photon_event<R>(A, p, s, G, sc);
+                alive = photon_event<R>(A, p, s, G, sc, b, out);
             else if (A.woodcock && G.g->wc.mu && s.split == 0u)
                 alive = photon_flight<R>(A, p, s, G, nsteps, ncross);
             else
@@ -1119,13 +1232,19 @@ __global__ void __launch_bounds__(256, Waves<R>::photon) k_photon(KArgs<R> A)
                 longest = max(longest, trips);
             }
         }
+        if (__ballot(out != 0u)) {
+            stage.push(A.qe, (out & OUT_MADE) != 0u, b, A.status);
+            stage.push(A.qe, (out & OUT_SELF) != 0u, p, A.status);
+        }
     }
+    stage.flush(A.qe, A.status);
     wave_max_to(A.longest, longest);
     sc.flush(G);
     if (nyield) atomicAdd(&A.status->yields, (unsigned long long)nyield);
     atomicAdd(&A.status->photon_steps, (unsigned long long)nsteps);
     atomicAdd(&A.status->photon_cross, (unsigned long long)ncross);
     atomicAdd(&A.status->photon_dep, (unsigned long long)sc.ndep);
+    events_end<false>(A.status);
 }
 
 template <typename R>
@@ -1143,7 +1262,8 @@ __global__ void __launch_bounds__(256, Waves<R>::electron) k_electron(KArgs<R> A
     Scorer<R> sc;
     uint32_t nsteps = 0, ncross = 0, trips = 0, here = 0, nyield = 0, longest = 0;
     const uint32_t in_end = min(*A.in_count, A.qin.cap);
-    const uint32_t yield_trips = in_end < A.drain_min ? min(A.yield_trips, A.yield_small) : A.yield_trips;
+    const uint32_t yield_trips = trips_per_launch(A, in_end);
+    Feed<FEED_ELECTRON> feed;
     bool alive = false, exhausted = (uint32_t)lane_id() >= lanes_used(in_end);
     for (;;) {
         // free lanes take new particles together (one counter atomic and one
@@ -1153,9 +1273,9 @@ __global__ void __launch_bounds__(256, Waves<R>::electron) k_electron(KArgs<R> A
         // only free lanes are active, and a ballot of `alive` there is 0)
         const unsigned long long want = __ballot(!alive && !exhausted);
         const bool none_live = __ballot(alive) == 0;
-        if (!alive && !exhausted && ((uint32_t)__popcll(want) >= A.fetch_min || none_live)) {
-            uint32_t i = wave_reserve(A.fetch, 1);
-            if (i < in_end) {
+        if (want != 0 && ((uint32_t)__popcll(want) >= A.fetch_min || none_live)) {
+            const uint32_t i = feed.take(A.fetch, in_end, want);
+            if (!alive && !exhausted && i < in_end) {
                 if (q_load(A.qin, i, p)) {
                     s.load(A.qin, i);
                     trips = A.qin.trips()[i];
@@ -1167,7 +1287,7 @@ __global__ void __launch_bounds__(256, Waves<R>::electron) k_electron(KArgs<R> A
                 find_voxel<R>(*G.g, p.ir, s.vox);
                 here = 0;
                 alive = true;
-            } else {
+            } else if (!alive) {
                 exhausted = true;
             }
         }
