@@ -100,6 +100,27 @@ __device__ __forceinline__ void ring_block(uint32_t b, uint32_t k0, uint32_t k1,
     for (int i = 0; i < 4; ++i) r[i * RNG_LANES] = philox_uniform(o[i]);
 }
 
+// Blocks b and, if `both`, b + 1, whose rounds share one key schedule and
+// overlap each other's multiplications.
+__device__ __forceinline__ void ring_two_blocks(uint32_t b, bool both, uint32_t k0, uint32_t k1, uint32_t col)
+{
+    uint32_t c0 = b, c1 = 0u, c2 = 0u, c3 = 0u, d0 = b + 1u, d1 = 0u, d2 = 0u, d3 = 0u;
+#pragma unroll
+    for (int r = 0; r < 10; ++r) {
+        if (r) { k0 += 0x9E3779B9u; k1 += 0xBB67AE85u; }
+        philox_round(c0, c1, c2, c3, k0, k1);
+        philox_round(d0, d1, d2, d3, k0, k1);
+    }
+    float *r = rng_ring + (b % RNG_RING) * (4 * RNG_LANES) + col;
+    r[0] = philox_uniform(c0); r[RNG_LANES] = philox_uniform(c1);
+    r[2 * RNG_LANES] = philox_uniform(c2); r[3 * RNG_LANES] = philox_uniform(c3);
+    if (both) {
+        r = rng_ring + ((b + 1u) % RNG_RING) * (4 * RNG_LANES) + col;
+        r[0] = philox_uniform(d0); r[RNG_LANES] = philox_uniform(d1);
+        r[2 * RNG_LANES] = philox_uniform(d2); r[3 * RNG_LANES] = philox_uniform(d3);
+    }
+}
+
 struct Rng {
     uint32_t k0, k1, ctr;
     uint32_t tail;           // draws [ctr, tail) are in this thread's ring column (multiple of 4)
@@ -237,12 +258,13 @@ __device__ __forceinline__ void ring_fill(Rng &r, bool live, uint64_t mask)
             if (j < n) ring_block<false>(first + j, k0, k1, col);
         tb += room;
     } else {
-        while (__popcll(__ballot(room != 0u)) >= OMC_RNG_FILL_LANES ||
+        while (__popcll(__ballot(room > 1u)) >= OMC_RNG_FILL_LANES ||
                __ballot(room > RNG_RING - OMC_RNG_FILL_MIN) != 0) {
             if (room) {
-                ring_block<false>(tb, r.k0, r.k1, threadIdx.x);
-                tb++;
-                room--;
+                const uint32_t n = min(room, 2u);
+                ring_two_blocks(tb, n == 2u, r.k0, r.k1, threadIdx.x);
+                tb += n;
+                room -= n;
             }
         }
     }
@@ -547,7 +569,9 @@ template <bool LANES> __device__ __forceinline__ void events_begin()
 __device__ __forceinline__ void count_event(int k) { atomicAdd(&ev_block[k], 1u); }
 
 // A frequent event of this thread's lane.
-__device__ __forceinline__ void count_lane_event(int k) { ev_lane[k - EV_NRARE][threadIdx.x] += 1u; }
+// (An LDS atomic without a result: a read, an addition and a write would wait
+// for the read.)
+__device__ __forceinline__ void count_lane_event(int k) { atomicAdd(&ev_lane[k - EV_NRARE][threadIdx.x], 1u); }
 
 // Adds the block's counts to the launch status (every thread of the block
 // calls it once, after its transport loop).

@@ -930,16 +930,7 @@ __device__ __forceinline__ int electron_iteration(const KArgs<R> &A, const MedRe
             call_howfar = false;
             do_single = false;
             called_msdist = true;
-            de = (R)eloss(csb, M.te, eke0, eke1, (double)rhof, (double)tustep, (double)range,
-                          (double)s.eke, (double)s.elke, s.lelke);
-            tvstep = tustep;
-            // msdist moves a copy; the original position is kept until
-            // after ausgab, which scores in the pre-step region
-            Particle<R> q = p;
-            count_lane_event(EV_MSDIST);
-            ustep = msdist<R>(T, M, q, imed, rhof, de, tustep, s.eke);
-            p.rng = q.rng;
-            xf = q.x; yf = q.y; zf = q.z; uf = q.u; vf = q.v; wf = q.w;
+            ustep = tustep;
         } else {
             called_msdist = false;
             R rnno = urand<R>(p.rng);
@@ -978,7 +969,30 @@ __device__ __forceinline__ int electron_iteration(const KArgs<R> &A, const MedRe
         howfar<R>(b, p.x, p.y, p.z, p.u, p.v, p.w, side, ustep);
     }
     if (ustep < (R)0) ustep = (R)0.0;
-    if (ustep == (R)0.0 || imed == -1) {
+    bool no_step = ustep == (R)0.0 || imed == -1;
+    const R rhof = s.rhof;
+    R vstep = ustep;
+    if (!no_step) {
+        // the energy loss of the step, for the three kinds of step together: the
+        // lanes of a wavefront that move by msdist, to a voxel side and within
+        // the voxel ran it one kind after the other before
+        tvstep = call_howfar ? vstep : tustep;
+        if (call_howfar && tvstep != tustep) do_single = false;
+        de = (R)eloss(csb, M.te, M.eke0, M.eke1, (double)rhof, (double)tvstep, (double)range, (double)s.eke,
+                      (double)s.elke, s.lelke);
+        if (called_msdist) {
+            // msdist moves a copy; the original position is kept until
+            // after ausgab, which scores in the pre-step region
+            Particle<R> q = p;
+            count_lane_event(EV_MSDIST);
+            ustep = msdist<R>(T, M, q, imed, rhof, de, tustep, s.eke);
+            p.rng = q.rng;
+            xf = q.x; yf = q.y; zf = q.z; uf = q.u; vf = q.v; wf = q.w;
+            if (ustep < (R)0) ustep = (R)0.0;
+            no_step = ustep == (R)0.0;
+        }
+    }
+    if (no_step) {
         if (ustep != (R)0.0) {
             R vstep = ustep;
             p.x += p.u * vstep;
@@ -996,19 +1010,6 @@ __device__ __forceinline__ int electron_iteration(const KArgs<R> &A, const MedRe
             return E_ALIVE;
         }
         return electron_interaction<R>(A, p, s);
-    }
-    R vstep = ustep;
-    const R rhof = s.rhof;
-    if (call_howfar) {
-        tvstep = vstep;
-        if (tvstep != tustep) do_single = false;
-        de = (R)eloss(csb, M.te, M.eke0, M.eke1, (double)rhof, (double)tvstep, (double)range,
-                      (double)s.eke, (double)s.elke, s.lelke);
-    } else {
-        tvstep = tustep;
-        if (!called_msdist)
-            de = (R)eloss(csb, M.te, M.eke0, M.eke1, (double)rhof, (double)tvstep, (double)range,
-                          (double)s.eke, (double)s.elke, s.lelke);
     }
     R edep = de;
     R ekef = s.eke - de;
