@@ -52,11 +52,12 @@ typedef struct {
     int64_t chunk;           /* live particles per pipeline before new primaries
                                 are held back; 0 = automatic */
     int     pipelines;       /* concurrent transport pipelines (streams),
-                                at most 16; 0 = automatic (6; the autotuner
-                                tries up to 12).  Each stream, and the context's
-                                helper stream, needs a hardware queue of its
-                                own: set GPU_MAX_HW_QUEUES >= pipelines + 1
-                                before HIP starts */
+                                at most 16; 0 = automatic (as many as get a
+                                hardware queue of their own, 4 to 6; the
+                                autotuner tries up to 12).  A pipeline that
+                                shares a queue with another runs after it:
+                                for more than 4, set GPU_MAX_HW_QUEUES >=
+                                pipelines + 1 before HIP starts */
     int     yield_trips;     /* transport loop trips a particle may take in
                                 one launch before it continues in the next
                                 (its lane state travels with it, so results

@@ -75,17 +75,18 @@ struct DevBuf {
 constexpr int MAX_JOBS = 4096;
 constexpr int MAX_SEGS = 512;
 constexpr int MAX_PIPES = 16;
-// Pipelines x chunk on the 64^3 slab phantom with the 6 MV spectrum (steps
-// of 1e8 histories, 16 hardware queues): the FP32 engine gains from
-// overlapping pipelines up to 10 (histories/s at 4M live particles each: 6
-// pipelines 2.15e8, 7 2.18e8, 8 2.28e8, 10 2.38e8, 12 2.38e8), while the
-// FP64 engine, whose charged-particle kernel holds 2 waves per SIMD, is flat
-// from 6 to 12 (1.07e8-1.09e8).  The default stays at 6 for both: the
-// serving loop has been exercised at 6, and the autotuner reaches 10-12
-// where a workload gains.  Each pipeline stream and the helper stream need
-// a hardware queue of their own (GPU_MAX_HW_QUEUES=16, which the drivers
-// set); pipelines that share a queue serialise.
+// Pipelines of a context that names no number: one per hardware queue, at
+// least 4 and at most 6.  With HIP's default of 4 queues (ms, 4 / 6
+// pipelines): FP32 slab of 1e8 histories 324-358 / 346, 400 beamlets 458 /
+// 479, five-beam plan 190 / 223, serving burst 141 / 156, 1e6 photons on a
+// graded grid 29 / 42, 5e6 FP64 slab histories 68 / 93: a pipeline that shares
+// a queue runs after the other one.  With 16 queues the FP32 engine gains up
+// to 10 pipelines and FP64 is flat from 6 on, but the serving loop has been
+// exercised at 6; the autotuner reaches 10-12 where a workload gains.
+constexpr int LEAST_PIPES = 4;
 constexpr int DEFAULT_PIPES = 6;
+constexpr int PROBE_US = 150;         // longest wait of the overlap probe
+constexpr int PROBE_MISSES = 8;       // streams in a row without a queue of their own that end the search
 constexpr int64_t DEFAULT_CHUNK = 1 << 22;
 // Batches of one work admitted batch by batch that may be in flight at once
 // (each is a job with its own grid).  Runs have held up to 13; a serving
@@ -264,6 +265,7 @@ struct omc_dev_ctx {
     hipStream_t aux = nullptr;    // admission and finishing work
     int64_t budget = 0;
     int64_t used = 0;
+    uint32_t *d_probe = nullptr;      // [2] flag and answer of the overlap probe
     void *scratch = nullptr;          // this device's scratch array (device address)
     int64_t tally_cap = 0;            // largest whole batch tally of a job (bytes; 0 = no limit)
     int64_t sort_min = 0;             // charged-particle launches of at least this many are energy-ordered (0 = never)
@@ -381,9 +383,64 @@ template <typename R> Queue<R> queue_view(const omc_dev_ctx *c, const Pipe &P, i
     return q;
 }
 
+// Whether work on two streams runs at the same time: a kernel on `a` waits (a
+// bounded time) for one on `b`, launched after it.  That one follows another on
+// `b`, so it is held back behind everything earlier in its hardware queue (two
+// streams' kernels may overlap within a queue while neither waits for one of
+// its own stream).
+int streams_overlap(omc_dev_ctx *c, hipStream_t a, hipStream_t b, bool *yes)
+{
+    uint32_t seen = 0;
+    launch_set_u32(c->d_probe, 2, 0u, a);
+    HIPCHK(hipStreamSynchronize(a));
+    launch_probe_wait(c->d_probe, PROBE_US, a);
+    launch_set_u32(c->d_probe, 1, 0u, b);
+    launch_set_u32(c->d_probe, 1, 1u, b);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(b));
+    HIPCHK(hipMemcpyAsync(&seen, c->d_probe + 1, sizeof seen, hipMemcpyDeviceToHost, a));
+    HIPCHK(hipStreamSynchronize(a));
+    *yes = seen != 0;
+    return OMC_OK;
+}
+
+// Streams for `most` pipelines.  The runtime maps streams onto a few hardware
+// queues (GPU_MAX_HW_QUEUES, 4 unless set) by its own count of their users,
+// and two pipelines on one queue run in turn.  Streams that overlap all those
+// chosen before are taken as long as the runtime gives some; the rest, up to
+// `least`, share.  The streams passed over stay until the end, so that the
+// next ones land on other queues.
+int pick_streams(omc_dev_ctx *c, int least, int most, std::vector<hipStream_t> &out)
+{
+    std::vector<hipStream_t> passed;
+    int rc = OMC_OK;
+    for (int misses = 0; !rc && (int)out.size() < most && misses < PROBE_MISSES;) {
+        hipStream_t s = nullptr;
+        if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) { rc = fail(OMC_EDEVICE, "stream"); break; }
+        bool apart = true;
+        for (size_t i = 0; !rc && apart && i < out.size(); ++i) rc = streams_overlap(c, out[i], s, &apart);
+        if (apart) misses = 0;
+        else ++misses;
+        (apart ? out : passed).push_back(s);
+    }
+    while (!rc && (int)out.size() < least) {
+        if (passed.empty()) {
+            hipStream_t s = nullptr;
+            if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) { rc = fail(OMC_EDEVICE, "stream"); break; }
+            passed.push_back(s);
+        }
+        out.push_back(passed.back());
+        passed.pop_back();
+    }
+    for (hipStream_t s : passed) (void)hipStreamDestroy(s);
+    if (rc)
+        for (hipStream_t s : out) (void)hipStreamDestroy(s);
+    if (rc) out.clear();
+    return rc;
+}
+
 template <typename R> int alloc_pipe(omc_dev_ctx *c, Pipe &P)
 {
-    if (hipStreamCreateWithFlags(&P.stream, hipStreamNonBlocking) != hipSuccess) return fail(OMC_EDEVICE, "stream");
     hipEvent_t *evs[] = { &P.ev_src0, &P.ev_src1, &P.ev_ph0, &P.ev_ph1, &P.ev_el0, &P.ev_el1, &P.ev_begin,
                           &P.ev_end[0], &P.ev_end[1] };
     for (auto *e : evs) HIPCHK(hipEventCreate(e));
@@ -1435,16 +1492,21 @@ static int64_t pipe_bytes(const omc_dev_ctx *c)
            MAX_SEGS * sizeof(SourceSeg) + sizeof(uint32_t) * SORT_BUCKETS * SORT_BLOCKS;
 }
 
-// (Re)builds the pipelines: npipes streams, each with queues four times
-// `chunk` deep (a generation's secondaries) and the sorted copy of a
-// charged-particle input; the five take at most half the budget, which can
-// lower the chunk.  No work may be queued.
+// (Re)builds the pipelines: npipes streams (0: as many as run side by side),
+// each with queues four times `chunk` deep (a generation's secondaries) and
+// the sorted copy of a charged-particle input; the five take at most half the
+// budget, which can lower the chunk.  No work may be queued.
 static int configure_pipes(omc_dev_ctx *c, int npipes, int64_t chunk)
 {
     for (auto &P : c->pipes) free_pipe(P);
     if (!c->pipes.empty()) c->used -= (int64_t)c->pipes.size() * pipe_bytes(c);
     c->pipes.clear();
-    npipes = std::max(1, std::min(npipes, MAX_PIPES));
+    npipes = std::min(npipes, MAX_PIPES);
+    std::vector<hipStream_t> streams;
+    OMC_TRY_DEV(pick_streams(c, npipes > 0 ? npipes : LEAST_PIPES, npipes > 0 ? npipes : DEFAULT_PIPES, streams));
+    npipes = (int)streams.size();
+    c->pipes.resize(npipes);
+    for (int p = 0; p < npipes; ++p) c->pipes[p].stream = streams[p];
     const size_t pb = c->precision == OMC_PREC_FP64 ? particle_bytes<double>() : particle_bytes<float>();
     c->chunk = chunk;
     int64_t cap = std::max<int64_t>(4 * c->chunk, 1 << 12);
@@ -1455,9 +1517,12 @@ static int configure_pipes(omc_dev_ctx *c, int npipes, int64_t chunk)
     }
     cap = std::min<int64_t>(cap, 1 << 26);
     c->chunk = std::min<int64_t>(c->chunk, cap / 4 > 0 ? cap / 4 : 1);
-    if (cap < 64) return fail(OMC_EBUDGET, "HBM budget %lld too small for the particle queues", (long long)c->budget);
+    if (cap < 64) {
+        for (auto &P : c->pipes) free_pipe(P);
+        c->pipes.clear();
+        return fail(OMC_EBUDGET, "HBM budget %lld too small for the particle queues", (long long)c->budget);
+    }
     c->qcap = (uint32_t)cap;
-    c->pipes.resize(npipes);
     for (auto &P : c->pipes) {
         const int rc = c->precision == OMC_PREC_FP64 ? alloc_pipe<double>(c, P) : alloc_pipe<float>(c, P);
         if (rc) return rc;
@@ -1510,7 +1575,8 @@ int omc_dev_create(omc_dev_ctx **out, const omc_dev_opts *opts)
     if (!rc) rc = dalloc(c, (void **)&c->d_jobs, MAX_JOBS * sizeof(DevJob));
     const size_t phb = o.precision == OMC_PREC_FP64 ? sizeof(DevPhantom<double>) : sizeof(DevPhantom<float>);
     if (!rc) rc = dalloc(c, &c->d_phantoms, MAX_PHANTOMS * phb);
-    if (!rc) rc = configure_pipes(c, o.pipelines > 0 ? o.pipelines : DEFAULT_PIPES, o.chunk > 0 ? o.chunk : DEFAULT_CHUNK);
+    if (!rc) rc = dalloc(c, (void **)&c->d_probe, 2 * sizeof(uint32_t));
+    if (!rc) rc = configure_pipes(c, o.pipelines, o.chunk > 0 ? o.chunk : DEFAULT_CHUNK);
     if (rc) { omc_dev_destroy(c); return rc; }
     *out = c;
     return OMC_OK;
@@ -1528,7 +1594,7 @@ int omc_dev_destroy(omc_dev_ctx *c)
     if (c->ev_fin) (void)hipEventDestroy(c->ev_fin);
     for (auto &kv : c->pool) (void)hipFree(kv.second);
     void *ptrs[] = { c->small, c->ph_mfp, c->ph_br, c->ph_pmax, c->el, c->csda, c->spin, c->ms,
-                     c->d_jobs, c->d_phantoms, c->fin_sums };
+                     c->d_jobs, c->d_phantoms, c->fin_sums, c->d_probe };
     for (void *p : ptrs) if (p) (void)hipFree(p);
     for (auto &P : c->ph) {
         DevBuf *bufs[] = { &P.xb, &P.yb, &P.zb, &P.sides, &P.med, &P.rhof, &P.rho, &P.wc };

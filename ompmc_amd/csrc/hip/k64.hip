@@ -163,6 +163,19 @@ __global__ void k_set_u32(uint32_t *p, int n, uint32_t v)
     if (i < n) p[i] = v;
 }
 
+// (wall_clock64 counts at 100 MHz; the wait also ends after a fixed number of
+// looks.)
+__global__ void k_probe_wait(uint32_t *flag, uint64_t ticks)
+{
+    const uint64_t t0 = wall_clock64();
+    uint32_t v = 0;
+    for (int look = 0; look < 100000 && !v && wall_clock64() - t0 < ticks; ++look) {
+        v = __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __builtin_amdgcn_s_sleep(4);
+    }
+    __hip_atomic_store(flag + 1, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 __global__ void k_zero_f64(double *p, int64_t n)
 {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -373,6 +386,11 @@ void launch_set_u32(uint32_t *p, int n, uint32_t v, hipStream_t st)
 {
     if (n <= 0) return;
     hipLaunchKernelGGL(k_set_u32, dim3((n + 255) / 256), dim3(256), 0, st, p, n, v);
+}
+
+void launch_probe_wait(uint32_t *flag, int us, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_probe_wait, dim3(1), dim3(1), 0, st, flag, (uint64_t)us * 100u);
 }
 
 void launch_zero_f64(double *p, int64_t n, hipStream_t st)

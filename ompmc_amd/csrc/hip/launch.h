@@ -52,6 +52,9 @@ void launch_fold(const double *tally, int nbatch, int64_t nreg, double *s, doubl
 void launch_accum(const double *grid, int64_t nreg, double *s, double *s2, hipStream_t st);
 void launch_set_u32(uint32_t *p, int n, uint32_t v, hipStream_t st);
 void launch_zero_f64(double *p, int64_t n, hipStream_t st);
+// Waits until flag[0] is set, at most `us` microseconds, and writes what it
+// saw to flag[1].
+void launch_probe_wait(uint32_t *flag, int us, hipStream_t st);
 
 // Start of a generation: zero the next generation's queue tails and both
 // fetch counters.  counts = [photon cur/next, charged cur/next, fetch x2].

@@ -1091,12 +1091,14 @@ template <typename R> __device__ __forceinline__ uint32_t trips_per_launch(const
 // Minimum waves per SIMD the register allocation of each transport kernel
 // must allow (the second __launch_bounds__ argument); values above what the
 // kernel needs make the compiler keep fewer values in VGPRs.  Chosen by
-// sweeps on the slab phantom: FP32 photon 4 (no spills) / electron 4 (128
-// VGPRs and a few spills; 3-4% more histories/s than 3 waves without
-// spills), FP64 photon 2 / electron 2 (a few spills, still faster than one
+// sweeps on the slab phantom: FP32 photon 3 (what the LDS of its staged
+// particles and rings allows; 4 spills registers and measures the same) /
+// electron 4 (128 VGPRs and a few spills; alone on the device 3 waves without
+// spills are faster, 81.3 against 84.3 ms per 2e7 histories, but with four
+// pipelines on it a slab of 1e8 takes 340 ms with 3 and 324 with 4), FP64 photon 2 / electron 2 (a few spills, still faster than one
 // wave).
 #ifndef OMC_WAVES_P32
-#define OMC_WAVES_P32 4
+#define OMC_WAVES_P32 3
 #endif
 #ifndef OMC_WAVES_E32
 #define OMC_WAVES_E32 4
