@@ -145,6 +145,26 @@ struct Rng {
         ctr = c + 1u;
         return rng_ring[(c % (4 * RNG_RING)) * RNG_LANES + threadIdx.x];
     }
+    // Makes the next n draws available to at() (n <= 4 * RNG_RING - 3).
+    __device__ __forceinline__ void ensure(uint32_t n)
+    {
+        const uint32_t end = ctr + n;
+        if (__ballot(end > tail) != 0) {
+            if (end > tail) {
+                uint32_t t = max(tail, ctr & ~3u);
+                do {
+                    ring_block<true>(t >> 2, k0, k1, threadIdx.x);
+                    t += 4u;
+                } while (t < end);
+                tail = t;
+            }
+        }
+    }
+    // Draw ctr + k, without taking it.
+    __device__ __forceinline__ float at(uint32_t k) const
+    {
+        return rng_ring[((ctr + k) % (4 * RNG_RING)) * RNG_LANES + threadIdx.x];
+    }
     // Key of a secondary: the Philox block (ctr, tag, 0, 0) under this key.
     // Interactions use tag 1 for the particles they create; tag 2 is for a
     // copy of the stream's own particle handed on while the stream goes on

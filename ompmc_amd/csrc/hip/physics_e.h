@@ -49,7 +49,22 @@ __device__ __forceinline__ double eloss(const ElecCsda *bins, double te, double 
         if (tuss <= 0) {
             de = eke - te * 0.99;
         } else {
-            while (lt > 0 && tuss < bins[lt].range) lt -= 1;
+            // down to the bin the residual range falls in, four bins' ranges at
+            // a time: one after the other, each step waited for its load (4.8
+            // passes a trip of a wavefront on the slab)
+            bool down = true;
+            while (down) {
+                const double r0 = bins[lt].range, r1 = bins[max(lt - 1, 0)].range, r2 = bins[max(lt - 2, 0)].range,
+                             r3 = bins[max(lt - 3, 0)].range;
+                down = lt > 0 && tuss < r0;
+                lt -= down;
+                down = down && lt > 0 && tuss < r1;
+                lt -= down;
+                down = down && lt > 0 && tuss < r2;
+                lt -= down;
+                down = down && lt > 0 && tuss < r3;
+                lt -= down;
+            }
             double elktmp = (lt + 2 - eke0) / eke1;
             double eketmp = bins[lt + 1].earr;
             tuss = (bins[lt + 1].range - tuss) / rhof;
@@ -314,7 +329,11 @@ __device__ __forceinline__ R msdist(const DevTables<R> &T, const MedRec<R> &M, P
     R c = eta * ((R)1.0 - delta);
     R w1v2 = w1 * v2;
     R ut = b * sint1 * cphi1 + c * (cphi1 * u2 - sphi1 * w1v2) + eta1 * us * temp1;
-    R vt = b * sint1 * sphi1 + c * (sphi1 * u2 + cphi1 * w1v2) + eta1 * vs * temp1;
+    // (which product of a sum the FP32 build fuses: see rounded)
+    R c1w1v2 = cphi1 * w1v2, bs1 = b * sint1 * sphi1;
+    rounded(c1w1v2);
+    rounded(bs1);
+    R vt = bs1 + c * (sphi1 * u2 + c1w1v2) + eta1 * vs * temp1;
     R wt = eta1 * ((R)1.0 + temp) + b * w1 + c * w2 + eta1 * ws * temp1;
     R ustep = tustep * m_sqrt(ut * ut + vt * vt + wt * wt);
 
@@ -452,7 +471,9 @@ __device__ void brems(const DevTables<R> &T, Particle<R> &a, Particle<R> &b, int
     if (sinpsi >= (R)1.0E-10) {
         R us = sinthe * cphi, vs = sinthe * sphi;
         b.u = Cc * cosdel * us - sindel * vs + A * costhe;
-        b.v = Cc * sindel * us + cosdel * vs + B * costhe;
+        R cv = cosdel * vs;
+        rounded(cv);
+        b.v = Cc * sindel * us + cv + B * costhe;
         b.w = Cc * costhe - sinpsi * us;
     } else {
         b.u = sinthe * cphi;
@@ -585,7 +606,9 @@ __device__ void annih(Particle<R> &a, Particle<R> &b)
         us = sinthe * cphi;
         vs = sinthe * sphi;
         a.u = cc * cosdel * us - sindel * vs + aa * costhe;
-        a.v = cc * sindel * us + cosdel * vs + bb * costhe;
+        R cv = cosdel * vs;
+        rounded(cv);
+        a.v = cc * sindel * us + cv + bb * costhe;
         a.w = cc * costhe - sinpsi * us;
     } else {
         a.u = sinthe * cphi;
@@ -602,7 +625,9 @@ __device__ void annih(Particle<R> &a, Particle<R> &b)
         us = sinthe * cphi;
         vs = sinthe * sphi;
         b.u = cc * cosdel * us - sindel * vs + aa * costhe;
-        b.v = cc * sindel * us + cosdel * vs + bb * costhe;
+        R cv = cosdel * vs;
+        rounded(cv);
+        b.v = cc * sindel * us + cv + bb * costhe;
         b.w = cc * costhe - sinpsi * us;
     } else {
         b.u = sinthe * cphi;
