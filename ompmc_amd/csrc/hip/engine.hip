@@ -94,22 +94,17 @@ constexpr int64_t DEFAULT_CHUNK = 1 << 22;
 // cause not yet found, so the count is held near the range that has run.
 constexpr int64_t MAX_SPLIT_INFLIGHT = 16;
 constexpr uint32_t DEFAULT_YIELD_TRIPS = 4096;
-// A launch whose input is below the drain threshold (it cannot fill the
-// device) but more than four particles to a wavefront hands its particles on
-// after this many trips: the photons that its
-// charged particles have made by then are followed while its longest tracks
-// go on, instead of after them, and the tracks left are spread over the
-// device again.  A generation costs about 0.2 ms, as much as 40 trips of a
-// lone particle.  One 2e4-history beamlet request on the patient phantom, FP32
-// / FP64: 18.9 / 27.5 ms at 4096 trips, 18.7 / 30.7 at 512, 20.2 / 34.5 at
-// 256; 1e6 photons on the graded 61^3 grid, FP32, 56 / 46 / 47 ms.
-constexpr uint32_t SMALL_YIELD_TRIPS = 512;
+// Particles x trips of a launch of middling size (trips_per_launch): it cannot
+// fill the device and hands its particles on early.  A generation costs
+// 0.2-0.5 ms.  ms at 512 trips / 2^24 / 2^23 / 2^22 particle-trips: 1e6 photons
+// on the graded 61^3 grid 27.9 / 28.0 / 26.7 / 26.4, 2e5 electrons 38.4 / 36.5 /
+// 37.6 / 35.0, 5e6 FP64 slab histories 64.3 / 65.3 / 63.1 / 65.1, 25 FP64
+// beamlets 47.3 / 48.3 / 46.2 / 48.5.
+constexpr uint32_t SMALL_TRIPS = 1u << 23;
 // Wavefronts per SIMD over which a small launch's particles are spread
-// (lanes_used).  A 1e3-photon FP64 call on the 40^3 water cube takes 8.7 ms
-// with 64 particles to a wavefront, 5.1-5.3 ms spread over 1, 2 or 4 per
-// SIMD; the FP32 beamlet request 22.5 ms against 18.7; with 4 per SIMD the
-// wavefronts of larger inputs (2e5 electrons, 1e6 photons) slow each other
-// down (5e6 FP64 slab histories 120 ms against 109 at 2).
+// (lanes_used) while it is the only one.  A 1e3-photon FP64 call on the 40^3
+// water cube takes 8.7 ms with 64 particles to a wavefront, 5.1-5.3 ms spread
+// over 1, 2 or 4 per SIMD; the FP32 beamlet request 22.5 ms against 18.7.
 constexpr int SPREAD_WAVES = 2;
 // Drain compaction: once a launch's input is used up, a wavefront with at
 // most 32 live lanes hands its particles (after 16 trips in the launch) to
@@ -117,6 +112,12 @@ constexpr int SPREAD_WAVES = 2;
 // 38 -> 55M histories/s, FP64 37 -> 42M).
 constexpr uint32_t DEFAULT_DRAIN_LANES = 32;
 constexpr uint32_t DEFAULT_DRAIN_TRIPS = 16;
+// Wavefronts per SIMD of the charged-particle kernel (its blocks per CU: one
+// wavefront of a block runs on each SIMD).
+constexpr int resident_waves(int precision)
+{
+    return precision == OMC_PREC_FP64 ? Waves<double>::electron : Waves<float>::electron;
+}
 // Repacking only pays while the device is full: a launch whose input is
 // smaller than the lanes the device holds resident (CUs x 4 SIMDs x the
 // electron kernel's waves per SIMD x 64) runs without draining.  A lone
@@ -124,7 +125,7 @@ constexpr uint32_t DEFAULT_DRAIN_TRIPS = 16;
 // handed on every 16 trips.
 constexpr int64_t drain_min_default(int cus, int precision)
 {
-    return (int64_t)cus * 4 * (precision == OMC_PREC_FP64 ? 2 : 4) * 64;
+    return (int64_t)cus * 4 * resident_waves(precision) * 64;
 }
 // A photon wavefront runs its waiting events (interaction, re-entry) once
 // half its live lanes wait for one (slab sweep of 2/4/8/16: 2 first, 22%
@@ -1123,12 +1124,25 @@ static int pull_segments(omc_dev_ctx *c, int pi, int64_t room, uint32_t &injP, u
     return nseg;
 }
 
-// Blocks of a transport launch over at most n particles.
+// Blocks of a transport launch over at most n particles.  No launch takes
+// more than 15/16 of the blocks the device holds resident: blocks beyond that
+// would only wait, and the other pipelines' small kernels (counters, flags,
+// copies, source) would wait behind them for a slot, up to 3.6 ms each
+// (serving burst 137 ms with twice the resident blocks, 129 with 15/16; FP32
+// slab of 1e8 histories 318 and 311).  A small launch spreads over SPREAD_WAVES
+// wavefronts per SIMD, or over its share of the device where other pipelines
+// are at work too (1e6 photons on a graded grid 30.5 ms without sharing, 27.9
+// with; 5e6 FP64 slab histories 66.6 and 64.3).
 static int transport_grid(const omc_dev_ctx *c, int64_t n)
 {
-    const int64_t full = (n + RNG_LANES - 1) / RNG_LANES, wide = (int64_t)c->cus * SPREAD_WAVES;
+    int active = 0;
+    for (const auto &P : c->pipes) active += P.inflight || P.nP || P.nE;
+    const int64_t resident = (int64_t)c->cus * resident_waves(c->precision), most = resident - resident / 16;
+    const int64_t share = std::max<int64_t>(c->cus / 2, most / std::max(active, 1));
+    const int64_t wide = std::min<int64_t>((int64_t)c->cus * SPREAD_WAVES, share);
+    const int64_t full = (n + RNG_LANES - 1) / RNG_LANES;
     const int64_t one = (n + RNG_LANES / 64 - 1) / (RNG_LANES / 64);      // one particle per wavefront
-    return (int)std::max<int64_t>(1, std::min<int64_t>((int64_t)c->cus * 8, std::max(full, std::min(one, wide))));
+    return (int)std::max<int64_t>(1, std::min(most, std::max(full, std::min(one, wide))));
 }
 
 template <typename R> static int launch_generation(omc_dev_ctx *c, int pi)
@@ -1165,7 +1179,7 @@ template <typename R> static int launch_generation(omc_dev_ctx *c, int pi)
     A.qp = queue_view<R>(c, P, nxt);
     A.status = P.d_status;
     A.yield_trips = c->yield_trips;
-    A.yield_small = SMALL_YIELD_TRIPS;
+    A.small_trips = SMALL_TRIPS;
     A.drain_lanes = c->drain_lanes;
     A.drain_trips = c->drain_trips;
     A.drain_min = (uint32_t)std::min<int64_t>(c->drain_min, UINT32_MAX);

@@ -32,7 +32,7 @@ template <typename R> struct KArgs {
     Queue<R> qe;             // charged-particle output queue
     DevStatus *status;
     uint32_t yield_trips;    // loop trips a particle may take per launch...
-    uint32_t yield_small;    // ...and in a launch of middling size (trips_per_launch)
+    uint32_t small_trips;    // ...and trips x particles of a launch of middling size (trips_per_launch)
     uint32_t drain_lanes;    // once the input is used up, a wave with at most
                              // this many live lanes hands its particles on...
     uint32_t drain_trips;    // ...if they have taken this many trips here...
@@ -1081,11 +1081,15 @@ __device__ __forceinline__ uint32_t lanes_used(uint32_t in_end)
 // Loop trips a particle may take in this launch.  A launch that cannot fill
 // the device (fewer than drain_min particles) hands its tracks on early, so
 // that the photons its charged particles made are followed meanwhile and the
-// tracks left are spread anew; with four or fewer particles to a wavefront
-// there is nothing left to spread, and the launch runs to its end.
+// tracks left are spread anew: the earlier the more particles it holds (most
+// of them end soon, and the rest sits in crowded wavefronts until then), 64
+// trips to 2048.  With four or fewer particles to a wavefront there is
+// nothing left to spread, and the launch runs to its end.
+constexpr uint32_t SMALL_TRIPS_LEAST = 64, SMALL_TRIPS_MOST = 2048, SMALL_LANES = 4;
 template <typename R> __device__ __forceinline__ uint32_t trips_per_launch(const KArgs<R> &A, uint32_t in_end)
 {
-    return in_end < A.drain_min && lanes_used(in_end) > 4u ? min(A.yield_trips, A.yield_small) : A.yield_trips;
+    if (in_end >= A.drain_min || lanes_used(in_end) <= SMALL_LANES) return A.yield_trips;
+    return min(A.yield_trips, min(max(A.small_trips / max(in_end, 1u), SMALL_TRIPS_LEAST), SMALL_TRIPS_MOST));
 }
 
 // Minimum waves per SIMD the register allocation of each transport kernel
