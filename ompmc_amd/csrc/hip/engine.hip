@@ -75,6 +75,9 @@ struct DevBuf {
 constexpr int MAX_JOBS = 4096;
 constexpr int MAX_SEGS = 512;
 constexpr int MAX_PIPES = 16;
+constexpr int JOB_STAGES = 64;        // jobs set up before the host waits for the set-ups
+constexpr size_t RESULT_KEEP = 32u << 20;   // result buffers up to this size are kept pinned
+constexpr int RESULT_BUFFERS = 2;
 // Pipelines of a context that names no number: one per hardware queue, at
 // least 4 and at most 6.  With HIP's default of 4 queues (ms, 4 / 6
 // pipelines): FP32 slab of 1e8 histories 324-358 / 346, 400 beamlets 458 /
@@ -184,6 +187,7 @@ struct Pipe {
     int cur = 0;
     uint32_t nP = 0, nE = 0;      // particles waiting in the current queues
     bool inflight = false;
+    bool jobs_new = false;        // jobs were admitted since its last generation
     bool had_src = false, had_ph = false, had_el = false;
     uint32_t injected = 0;        // primaries injected by the generation in flight
     uint32_t in_e = 0;            // charged particles in its queue at launch (known to the host)
@@ -222,6 +226,10 @@ struct Work {
     int job = -1;
     double submit_ms = 0, admit_ms = 0, finish_ms = 0;
     std::vector<double> sum, sum2;
+    // A finished request's sums [sum | sum of squares] where a pinned result
+    // buffer was free, else in the vectors above.
+    double *res = nullptr;
+    int64_t res_cap = 0;          // regions res has room for
 };
 
 // Where a synchronous run wants its results.
@@ -303,6 +311,16 @@ struct omc_dev_ctx {
     int64_t *h_rows = nullptr;        // [nvox]
     double *h_vals = nullptr;         // [nvox]
     uint32_t *h_nnz = nullptr;
+    // result buffers of requests, pinned: the sums are copied into one by the
+    // device and out of it by the poll, without a vector between
+    struct ResultBuf { double *p; int64_t cap; };
+    std::vector<ResultBuf> results;   // free ones
+    int64_t result_cap = 0;           // regions they have room for (0: none are kept)
+    // job set-up
+    struct JobStage { DevJob job; double cdf[2 * OMC_INVDIM]; };
+    JobStage *h_stage = nullptr;      // [JOB_STAGES] pinned
+    int staged = 0;                   // entries in use since the last wait
+    hipEvent_t ev_admit = nullptr;    // set-up of the jobs admitted so far
     std::deque<int> finishing;        // jobs whose results are being collected, oldest first
     hipEvent_t ev_fin = nullptr;      // end of the head job's current finishing stage
     // jobs
@@ -698,6 +716,18 @@ static int grow_finish_scratch(omc_dev_ctx *c, int64_t nvox)
     c->h_vals = (double *)h;                h += up(vals);
     c->h_nnz = (uint32_t *)h;
     c->fin_nvox = nvox;
+    for (auto &r : c->results) (void)hipHostFree(r.p);
+    c->results.clear();
+    c->result_cap = 0;
+    if (sums <= RESULT_KEEP) {
+        for (int i = 0; i < RESULT_BUFFERS; ++i) {
+            double *r = nullptr;
+            if (hipHostMalloc((void **)&r, sums, hipHostMallocDefault) != hipSuccess)
+                return fail(OMC_EDEVICE, "pinned result buffers (%zu bytes)", sums);
+            c->results.push_back({ r, nvox + 1 });
+        }
+        c->result_cap = nvox + 1;
+    }
     return OMC_OK;
 }
 
@@ -779,13 +809,16 @@ template <typename R> static int upload_phantom(omc_dev_ctx *c, const omc_phanto
 }
 
 // -------------------------------------------------------------- scheduler --
+// Bytes of a job's pooled buffer: its grids and, at the end, its spectrum.
+static size_t job_bytes(size_t tally_bytes)
+{
+    return ((tally_bytes + 255) & ~(size_t)255) + 2 * OMC_INVDIM * sizeof(double);
+}
+
 static void release_job(omc_dev_ctx *c, int j)
 {
     JobRec &J = c->jobs[j];
-    if (!J.borrowed) {
-        pool_free(c, J.tally, J.tally_bytes);
-        if (J.cdf) dfree(c, J.cdf, 2 * OMC_INVDIM * sizeof(double));
-    }
+    if (!J.borrowed) pool_free(c, J.tally, job_bytes(J.tally_bytes));
     if (J.ledger) dfree(c, J.ledger, J.ledger_bytes);
     J = JobRec();
     while (c->jobs_hi > 0 && !c->jobs[c->jobs_hi - 1].used) c->jobs_hi--;
@@ -796,7 +829,7 @@ static void end_work(omc_dev_ctx *c, Work *w, int status)
     // a work admitted batch by batch has several jobs but ends once
     if (w->state == W_DONE || w->state == W_FAILED) return;
     if (w->acc) {
-        dfree(c, w->acc, 2 * sizeof(double) * (size_t)w->nreg);
+        pool_free(c, w->acc, 2 * sizeof(double) * (size_t)w->nreg);
         w->acc = nullptr;
     }
     w->state = status == OMC_OK ? W_DONE : W_FAILED;
@@ -831,7 +864,7 @@ static int any_running(const omc_dev_ctx *c)
 // fit even with nothing else admitted fails with OMC_EBUDGET.  A work
 // admitted batch by batch stays in line until its last batch is admitted;
 // while its batches in flight are at its limit, the works behind it go on.
-static int admit(omc_dev_ctx *c)
+static int admit_works(omc_dev_ctx *c, bool &fresh)
 {
     size_t at = 0;
     while (at < c->waiting.size()) {
@@ -858,7 +891,7 @@ static int admit(omc_dev_ctx *c)
         J.tally_bytes = sizeof(double) * (size_t)w->nreg * slots;
         int rc = OMC_OK;
         if (split && !w->acc) {
-            rc = dalloc(c, (void **)&w->acc, 2 * sizeof(double) * (size_t)w->nreg);
+            rc = pool_alloc(c, (void **)&w->acc, 2 * sizeof(double) * (size_t)w->nreg);
             if (!rc) launch_zero_f64(w->acc, 2 * w->nreg, c->aux);
         }
         if (!rc && w->scratch) {
@@ -867,8 +900,9 @@ static int admit(omc_dev_ctx *c)
             J.tally = (double *)c->scratch;
             J.cdf = (double *)((char *)c->scratch + ((J.tally_bytes + 255) & ~(size_t)255));
         } else if (!rc) {
-            rc = pool_alloc(c, (void **)&J.tally, J.tally_bytes);
-            if (!rc) rc = dalloc(c, (void **)&J.cdf, 2 * OMC_INVDIM * sizeof(double));
+            // grids and spectrum in one buffer of the pool
+            rc = pool_alloc(c, (void **)&J.tally, job_bytes(J.tally_bytes));
+            if (!rc) J.cdf = (double *)((char *)J.tally + job_bytes(J.tally_bytes)) - 2 * OMC_INVDIM;
         }
         if (!rc && w->ledger) {
             J.ledger_bytes = sizeof(double) * OMC_LEDGER * (size_t)jn;
@@ -893,10 +927,14 @@ static int admit(omc_dev_ctx *c)
         const int64_t npipes = (int64_t)c->pipes.size();
         J.quantum = w->ticket >= 0 ? std::max<int64_t>(4096, c->chunk / 8)
                                    : std::max<int64_t>(65536, (jn + npipes - 1) / npipes);
-        launch_zero_f64(J.tally, w->nreg * slots, c->aux);
         if (J.ledger) launch_zero_f64(J.ledger, OMC_LEDGER * jn, c->aux);
-        HIPCHK(hipMemcpyAsync(J.cdf, w->cdf.data(), 2 * OMC_INVDIM * sizeof(double), hipMemcpyHostToDevice, c->aux));
-        DevJob d = w->tmpl;
+        if (c->staged == JOB_STAGES) {
+            HIPCHK(hipStreamSynchronize(c->aux));
+            c->staged = 0;
+        }
+        omc_dev_ctx::JobStage &stage = c->h_stage[c->staged++];
+        DevJob &d = stage.job;
+        d = w->tmpl;
         d.phantom = w->phantom;
         d.cdf1 = J.cdf;
         d.cdf2 = J.cdf + OMC_INVDIM;
@@ -907,8 +945,12 @@ static int admit(omc_dev_ctx *c)
         if (split) d.hist0 = w->tmpl.hist0 + (uint64_t)J.batch * (uint64_t)w->nperbatch;
         d.tally = J.tally;
         d.ledger = J.ledger;
-        HIPCHK(hipMemcpyAsync(c->d_jobs + slot, &d, sizeof d, hipMemcpyHostToDevice, c->aux));
-        HIPCHK(hipStreamSynchronize(c->aux));
+        const int ncdf = d.spectrum ? 2 * OMC_INVDIM : 0;
+        std::copy(w->cdf.begin(), w->cdf.begin() + ncdf, stage.cdf);
+        launch_job_setup(&d, c->d_jobs + slot, stage.cdf, J.cdf, ncdf, J.tally, w->nreg * slots, c->aux);
+        HIPCHK(hipGetLastError());
+        for (auto &P : c->pipes) P.jobs_new = true;
+        fresh = true;
         c->jobs_hi = std::max(c->jobs_hi, slot + 1);
         w->job = slot;
         if (w->state == W_WAITING) {
@@ -925,6 +967,16 @@ static int admit(omc_dev_ctx *c)
     return OMC_OK;
 }
 
+// The pipelines wait for the set-up on their own streams, so the scheduler does
+// not wait for it (behind whatever shares the helper stream's hardware queue).
+static int admit(omc_dev_ctx *c)
+{
+    bool fresh = false;
+    const int rc = admit_works(c, fresh);
+    if (fresh) HIPCHK(hipEventRecord(c->ev_admit, c->aux));
+    return rc;
+}
+
 // Finishing a job: its last particle is gone, so its tally is final.  The
 // results are collected on the helper stream while the pipelines go on:
 //   FIN_FOLD    fold the batches (accumEndep, omc_dosxyz.c:696-717) and/or
@@ -939,10 +991,34 @@ static bool wants_sums(const Work *w)
     return !k || k->sum || !k->beamlets;
 }
 
+// Where the sums of a work are copied to: a request's own result buffer where
+// one is free, else the shared pinned buffer.
+static double *sums_target(omc_dev_ctx *c, Work *w)
+{
+    if (w->sink || w->res) return w->res ? w->res : c->h_sums;
+    if (w->nreg <= c->result_cap && !c->results.empty()) {
+        w->res = c->results.back().p;
+        w->res_cap = c->results.back().cap;
+        c->results.pop_back();
+        return w->res;
+    }
+    return c->h_sums;
+}
+
+// Gives a request's result buffer back (one that was made for smaller
+// phantoms than are resident now is freed).
+static void give_back_result(omc_dev_ctx *c, Work *w)
+{
+    if (!w->res) return;
+    if (w->res_cap == c->result_cap && (int)c->results.size() < RESULT_BUFFERS) c->results.push_back({ w->res, w->res_cap });
+    else (void)hipHostFree(w->res);
+    w->res = nullptr;
+}
+
 static int finish_fold(omc_dev_ctx *c, int j)
 {
     JobRec &J = c->jobs[j];
-    const Work *w = J.w;
+    Work *w = J.w;
     const RunSink *k = w->sink;
     const int64_t nreg = w->nreg;
     hipStream_t s = c->aux;
@@ -952,13 +1028,13 @@ static int finish_fold(omc_dev_ctx *c, int j)
         if (w->acc) {
             launch_accum(J.tally, nreg, w->acc, w->acc + nreg, s);
             if (w->batches_done + 1 == w->nbatch &&
-                hipMemcpyAsync(c->h_sums, w->acc, 2 * (size_t)nreg * sizeof(double), hipMemcpyDeviceToHost, s) !=
+                hipMemcpyAsync(sums_target(c, w), w->acc, 2 * (size_t)nreg * sizeof(double), hipMemcpyDeviceToHost, s) !=
                     hipSuccess)
                 return fail(OMC_EDEVICE, "copy tallies");
         }
     } else if (wants_sums(w)) {
         launch_fold(J.tally, w->nbatch, nreg, c->fin_sums, c->fin_sums + nreg, s);
-        if (hipMemcpyAsync(c->h_sums, c->fin_sums, 2 * (size_t)nreg * sizeof(double), hipMemcpyDeviceToHost, s) !=
+        if (hipMemcpyAsync(sums_target(c, w), c->fin_sums, 2 * (size_t)nreg * sizeof(double), hipMemcpyDeviceToHost, s) !=
             hipSuccess)
             return fail(OMC_EDEVICE, "copy tallies");
     }
@@ -1002,7 +1078,9 @@ static int finish_deliver(omc_dev_ctx *c, int j)
     const bool last = J.batch < 0 || w->batches_done + 1 == w->nbatch;
     if (last && wants_sums(w)) {
         const double *h = c->h_sums;
-        if (!k) {
+        if (!k && w->res) {
+            // the poll copies them from there
+        } else if (!k) {
             w->sum.assign(h, h + nreg);
             w->sum2.assign(h + nreg, h + 2 * nreg);
         } else if (k->sum) {
@@ -1157,11 +1235,15 @@ template <typename R> static int launch_generation(omc_dev_ctx *c, int pi)
     const uint32_t inP = P.nP + injP, inE = P.nE + injE;
     if (!inP && !inE) return OMC_OK;
     HIPCHK(hipEventRecord(P.ev_begin, s));
-    launch_gen_reset(P.d_counts, nxt, s);
+    if (P.jobs_new) {
+        HIPCHK(hipStreamWaitEvent(s, c->ev_admit, 0));
+        P.jobs_new = false;
+    }
+    const int njobs = std::max(c->jobs_hi, 1);
+    launch_gen_begin(P.d_counts, nxt, P.d_flags, njobs, P.h->segs, P.d_segs, nseg, s);
     const Queue<R> qpc = queue_view<R>(c, P, P.cur), qec = queue_view<R>(c, P, 2 + P.cur);
     P.had_src = nseg > 0;
     if (P.had_src) {
-        HIPCHK(hipMemcpyAsync(P.d_segs, P.h->segs, nseg * sizeof(SourceSeg), hipMemcpyHostToDevice, s));
         HIPCHK(hipEventRecord(P.ev_src0, s));
         Launch<R>::source(c->d_jobs, (const DevPhantom<R> *)c->d_phantoms, P.d_segs, nseg, ntot, qpc, qec,
                           inP, inE, P.d_status, s);
@@ -1220,13 +1302,10 @@ template <typename R> static int launch_generation(omc_dev_ctx *c, int pi)
         HIPCHK(hipEventRecord(P.ev_el1, s));
     }
     HIPCHK(hipGetLastError());
-    const int njobs = std::max(c->jobs_hi, 1);
-    launch_set_u32(P.d_flags, njobs, 0u, s);
     const Queue<R> qpn = queue_view<R>(c, P, nxt), qen = queue_view<R>(c, P, 2 + nxt);
     launch_job_flags(qpn.meta(), qpn.count, qen.meta(), qen.count, c->qcap, P.d_flags, njobs, s);
-    HIPCHK(hipMemcpyAsync(P.h->counts, P.d_counts, 8 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipMemcpyAsync(&P.h->status, P.d_status, sizeof(DevStatus), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipMemcpyAsync(P.h->flags, P.d_flags, njobs * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+    launch_gen_end(P.d_counts, P.d_status, P.d_flags, njobs, P.h->counts, &P.h->status, P.h->flags, s);
+    HIPCHK(hipGetLastError());
     HIPCHK(hipEventRecord(P.ev_end[P.gen & 1], s));
     P.injected = ntot;
     P.inflight = true;
@@ -1586,6 +1665,10 @@ int omc_dev_create(omc_dev_ctx **out, const omc_dev_opts *opts)
     int rc = OMC_OK;
     if (hipStreamCreateWithFlags(&c->aux, hipStreamNonBlocking) != hipSuccess) rc = fail(OMC_EDEVICE, "stream");
     if (!rc && hipEventCreateWithFlags(&c->ev_fin, hipEventDisableTiming) != hipSuccess) rc = fail(OMC_EDEVICE, "event");
+    if (!rc && hipEventCreateWithFlags(&c->ev_admit, hipEventDisableTiming) != hipSuccess) rc = fail(OMC_EDEVICE, "event");
+    if (!rc && hipHostMalloc((void **)&c->h_stage, JOB_STAGES * sizeof(omc_dev_ctx::JobStage), hipHostMallocDefault) !=
+                   hipSuccess)
+        rc = fail(OMC_EDEVICE, "pinned job staging");
     if (!rc) rc = dalloc(c, (void **)&c->d_jobs, MAX_JOBS * sizeof(DevJob));
     const size_t phb = o.precision == OMC_PREC_FP64 ? sizeof(DevPhantom<double>) : sizeof(DevPhantom<float>);
     if (!rc) rc = dalloc(c, &c->d_phantoms, MAX_PHANTOMS * phb);
@@ -1605,7 +1688,10 @@ int omc_dev_destroy(omc_dev_ctx *c)
     c->finishing.clear();
     for (int j = 0; j < c->jobs_hi; ++j) if (c->jobs[j].used) release_job(c, j);
     if (c->h_sums) (void)hipHostFree(c->h_sums);
+    if (c->h_stage) (void)hipHostFree(c->h_stage);
     if (c->ev_fin) (void)hipEventDestroy(c->ev_fin);
+    if (c->ev_admit) (void)hipEventDestroy(c->ev_admit);
+    for (auto &r : c->results) (void)hipHostFree(r.p);
     for (auto &kv : c->pool) (void)hipFree(kv.second);
     void *ptrs[] = { c->small, c->ph_mfp, c->ph_br, c->ph_pmax, c->el, c->csda, c->spin, c->ms,
                      c->d_jobs, c->d_phantoms, c->fin_sums, c->d_probe };
@@ -1616,6 +1702,7 @@ int omc_dev_destroy(omc_dev_ctx *c)
     }
     for (auto &kv : c->tickets) {
         if (kv.second->acc) (void)hipFree(kv.second->acc);
+        if (kv.second->res) (void)hipHostFree(kv.second->res);
         delete kv.second;
     }
     if (c->aux) (void)hipStreamDestroy(c->aux);
@@ -2201,9 +2288,11 @@ int omc_dev_poll(omc_dev_ctx *c, int ticket, omc_dev_result *res, double *sum, d
     res->nhist = w->nhist;
     if (!res->done) return OMC_OK;
     if (w->state == W_DONE) {
-        if (sum) std::copy(w->sum.begin(), w->sum.end(), sum);
-        if (sum2) std::copy(w->sum2.begin(), w->sum2.end(), sum2);
+        const double *s1 = w->res ? w->res : w->sum.data(), *s2 = w->res ? w->res + w->nreg : w->sum2.data();
+        if (sum) std::copy(s1, s1 + w->nreg, sum);
+        if (sum2) std::copy(s2, s2 + w->nreg, sum2);
     }
+    give_back_result(c, w);
     c->tickets.erase(it);
     delete w;
     return OMC_OK;

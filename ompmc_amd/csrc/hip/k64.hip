@@ -1,5 +1,7 @@
 // FP64 transport kernels (built with FMA contraction off so that every
 // operation rounds as in the CPU reference).
+#include <algorithm>
+
 #include "kernels_impl.h"
 
 namespace omc {
@@ -183,16 +185,42 @@ __global__ void k_zero_f64(double *p, int64_t n)
     for (; i < n; i += stride) p[i] = 0.0;
 }
 
-__global__ void k_gen_reset(uint32_t *counts, int nxt)
+// Bookkeeping of a generation in one kernel before it and one after it: as a
+// kernel, a fill and up to four copies (a blit kernel each) it was five more
+// packets on the stream, 25 us at best and a wait for a free slot each while
+// other pipelines fill the device.
+__device__ __forceinline__ void copy_words(uint32_t *dst, const uint32_t *src, int n)
 {
-    if (threadIdx.x == 0) {
-        counts[nxt] = 0u;
-        counts[2 + nxt] = 0u;
-        counts[4] = 0u;
-        counts[5] = 0u;
-        counts[6] = 0u;         // longest charged-particle track of the generation
-        counts[7] = 0u;         // longest photon track
-    }
+    for (int i = threadIdx.x; i < n; i += blockDim.x) dst[i] = src[i];
+}
+
+__global__ void __launch_bounds__(256) k_gen_begin(uint32_t *counts, int nxt, uint32_t *flags, int njobs,
+                                                   const uint32_t *host_segs, uint32_t *segs, int nwords)
+{
+    // tails of the next queues, fetch counters, longest tracks
+    if (threadIdx.x < 8 && (threadIdx.x >= 4 || (int)(threadIdx.x & 1u) == nxt)) counts[threadIdx.x] = 0u;
+    for (int i = threadIdx.x; i < njobs; i += blockDim.x) flags[i] = 0u;
+    copy_words(segs, host_segs, nwords);
+}
+
+__global__ void __launch_bounds__(256) k_gen_end(const uint32_t *counts, const uint32_t *status, const uint32_t *flags,
+                                                 int njobs, uint32_t *host_counts, uint32_t *host_status,
+                                                 uint32_t *host_flags)
+{
+    copy_words(host_counts, counts, 8);
+    copy_words(host_status, status, (int)(sizeof(DevStatus) / 4));
+    copy_words(host_flags, flags, njobs);
+}
+
+// One job set up by one kernel (a fill and two copies from pageable memory
+// with a wait for them before).
+__global__ void __launch_bounds__(256) k_job_setup(const uint32_t *host_job, uint32_t *job, const double *host_cdf,
+                                                   double *cdf, int ncdf, double *tally, int64_t ntally)
+{
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
+    if (blockIdx.x == 0) copy_words(job, host_job, (int)(sizeof(DevJob) / 4));
+    for (int64_t i = t; i < ncdf; i += stride) cdf[i] = host_cdf[i];
+    for (int64_t i = t; i < ntally; i += stride) tally[i] = 0.0;
 }
 
 // One flag store per distinct job in a wavefront: lanes holding the same job
@@ -358,9 +386,28 @@ void launch_beamlet_column(const double *tally, int nslots, int nbatch, int isiz
                        S.vals);
 }
 
-void launch_gen_reset(uint32_t *counts, int nxt, hipStream_t st)
+void launch_gen_begin(uint32_t *counts, int nxt, uint32_t *flags, int njobs, const SourceSeg *host_segs,
+                      SourceSeg *segs, int nseg, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_gen_reset, dim3(1), dim3(64), 0, st, counts, nxt);
+    static_assert(sizeof(SourceSeg) % 4 == 0 && sizeof(DevStatus) % 4 == 0 && sizeof(DevJob) % 4 == 0, "word copies");
+    hipLaunchKernelGGL(k_gen_begin, dim3(1), dim3(256), 0, st, counts, nxt, flags, njobs, (const uint32_t *)host_segs,
+                       (uint32_t *)segs, (int)(nseg * sizeof(SourceSeg) / 4));
+}
+
+void launch_gen_end(const uint32_t *counts, const DevStatus *status, const uint32_t *flags, int njobs,
+                    uint32_t *host_counts, DevStatus *host_status, uint32_t *host_flags, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_gen_end, dim3(1), dim3(256), 0, st, counts, (const uint32_t *)status, flags, njobs,
+                       host_counts, (uint32_t *)host_status, host_flags);
+}
+
+void launch_job_setup(const DevJob *host_job, DevJob *job, const double *host_cdf, double *cdf, int ncdf,
+                      double *tally, int64_t ntally, hipStream_t st)
+{
+    const int64_t n = std::max<int64_t>(ntally, ncdf);
+    const int64_t blocks = std::min<int64_t>(std::max<int64_t>((n + 255) / 256, 1), 65536);
+    hipLaunchKernelGGL(k_job_setup, dim3((unsigned)blocks), dim3(256), 0, st, (const uint32_t *)host_job,
+                       (uint32_t *)job, host_cdf, cdf, ncdf, tally, ntally);
 }
 
 void launch_job_flags(const uint32_t *meta_p, const uint32_t *count_p, const uint32_t *meta_e,

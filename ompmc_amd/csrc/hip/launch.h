@@ -56,9 +56,22 @@ void launch_zero_f64(double *p, int64_t n, hipStream_t st);
 // saw to flag[1].
 void launch_probe_wait(uint32_t *flag, int us, hipStream_t st);
 
-// Start of a generation: zero the next generation's queue tails and both
-// fetch counters.  counts = [photon cur/next, charged cur/next, fetch x2].
-void launch_gen_reset(uint32_t *counts, int nxt, hipStream_t st);
+// Start of a generation: zero the next generation's queue tails, both fetch
+// counters and the flags of njobs jobs, and copy the source segments from the
+// pinned host table.  counts = [photon cur/next, charged cur/next, fetch x2,
+// longest tracks x2].
+void launch_gen_begin(uint32_t *counts, int nxt, uint32_t *flags, int njobs, const SourceSeg *host_segs,
+                      SourceSeg *segs, int nseg, hipStream_t st);
+
+// End of a generation: counters, status and job flags into the pipeline's
+// pinned mirror.
+void launch_gen_end(const uint32_t *counts, const DevStatus *status, const uint32_t *flags, int njobs,
+                    uint32_t *host_counts, DevStatus *host_status, uint32_t *host_flags, hipStream_t st);
+
+// A job's set-up from pinned host memory: its record, its spectrum (ncdf
+// values) and its zeroed grids (ntally values).
+void launch_job_setup(const DevJob *host_job, DevJob *job, const double *host_cdf, double *cdf, int ncdf,
+                      double *tally, int64_t ntally, hipStream_t st);
 
 // flags[j] = 1 for every job j that owns a particle in either queue
 // (meta[] >> 3), over the first min(*count, cap) entries; flags must be
