@@ -74,6 +74,7 @@ struct DevBuf {
 
 constexpr int MAX_JOBS = 4096;
 constexpr int MAX_SEGS = 512;
+constexpr size_t COUNT_BYTES = 8 * COUNT_STRIDE * sizeof(uint32_t);
 constexpr int MAX_PIPES = 16;
 constexpr int JOB_STAGES = 64;        // jobs set up before the host waits for the set-ups
 constexpr size_t RESULT_KEEP = 32u << 20;   // result buffers up to this size are kept pinned
@@ -172,8 +173,8 @@ struct PipeMirror {
 struct Pipe {
     hipStream_t stream = nullptr;
     void *q[4] = {};              // particle queues: photon cur/next, charged cur/next
-    uint32_t *d_counts = nullptr; // 4 tails + 2 fetch counters
-    DevStatus *d_status = nullptr;
+    uint32_t *d_counts = nullptr; // 4 tails, 2 fetch counters, 2 longest tracks (launch_gen_begin)
+    DevStatus *d_status = nullptr; // [STATUS_COPIES]
     uint32_t *d_flags = nullptr;  // [MAX_JOBS]
     SourceSeg *d_segs = nullptr;  // [MAX_SEGS]
     void *d_sorted = nullptr;     // [qcap] records: a charged-particle launch's input by falling energy
@@ -397,7 +398,7 @@ template <typename R> Queue<R> queue_view(const omc_dev_ctx *c, const Pipe &P, i
 {
     Queue<R> q;
     q.base = (char *)P.q[k];
-    q.count = P.d_counts + k;
+    q.count = P.d_counts + k * COUNT_STRIDE;
     q.cap = c->qcap;
     return q;
 }
@@ -464,16 +465,16 @@ template <typename R> int alloc_pipe(omc_dev_ctx *c, Pipe &P)
                           &P.ev_end[0], &P.ev_end[1] };
     for (auto *e : evs) HIPCHK(hipEventCreate(e));
     for (int k = 0; k < 4; ++k) OMC_TRY_DEV(dalloc(c, &P.q[k], particle_bytes<R>() * (size_t)c->qcap));
-    OMC_TRY_DEV(dalloc(c, (void **)&P.d_counts, 8 * sizeof(uint32_t)));
-    OMC_TRY_DEV(dalloc(c, (void **)&P.d_status, sizeof(DevStatus)));
+    OMC_TRY_DEV(dalloc(c, (void **)&P.d_counts, COUNT_BYTES));
+    OMC_TRY_DEV(dalloc(c, (void **)&P.d_status, STATUS_COPIES * sizeof(DevStatus)));
     OMC_TRY_DEV(dalloc(c, (void **)&P.d_flags, MAX_JOBS * sizeof(uint32_t)));
     OMC_TRY_DEV(dalloc(c, (void **)&P.d_segs, MAX_SEGS * sizeof(SourceSeg)));
     OMC_TRY_DEV(dalloc(c, &P.d_sorted, particle_bytes<R>() * (size_t)c->qcap));
     OMC_TRY_DEV(dalloc(c, (void **)&P.d_sort, sizeof(uint32_t) * SORT_BUCKETS * SORT_BLOCKS));
     HIPCHK(hipHostMalloc((void **)&P.h, sizeof(PipeMirror), hipHostMallocDefault));
     memset(P.h, 0, sizeof(PipeMirror));
-    HIPCHK(hipMemset(P.d_counts, 0, 8 * sizeof(uint32_t)));
-    HIPCHK(hipMemset(P.d_status, 0, sizeof(DevStatus)));
+    HIPCHK(hipMemset(P.d_counts, 0, COUNT_BYTES));
+    HIPCHK(hipMemset(P.d_status, 0, STATUS_COPIES * sizeof(DevStatus)));
     memset(&P.base, 0, sizeof P.base);
     return OMC_OK;
 }
@@ -1273,9 +1274,9 @@ template <typename R> static int launch_generation(omc_dev_ctx *c, int pi)
     if (P.had_ph) {
         A.qin = qpc;
         A.qe = qec;
-        A.in_count = P.d_counts + P.cur;
-        A.fetch = P.d_counts + 4;
-        A.longest = P.d_counts + 7;
+        A.in_count = P.d_counts + P.cur * COUNT_STRIDE;
+        A.fetch = P.d_counts + 4 * COUNT_STRIDE;
+        A.longest = P.d_counts + 7 * COUNT_STRIDE;
         HIPCHK(hipEventRecord(P.ev_ph0, s));
         Launch<R>::photon(A, transport_grid(c, inP), s);
         HIPCHK(hipEventRecord(P.ev_ph1, s));
@@ -1286,9 +1287,9 @@ template <typename R> static int launch_generation(omc_dev_ctx *c, int pi)
         // photon; lanes fetch until the queue's final count either way
         A.qin = qec;
         A.qe = queue_view<R>(c, P, 2 + nxt);
-        A.in_count = P.d_counts + 2 + P.cur;
-        A.fetch = P.d_counts + 5;
-        A.longest = P.d_counts + 6;
+        A.in_count = P.d_counts + (2 + P.cur) * COUNT_STRIDE;
+        A.fetch = P.d_counts + 5 * COUNT_STRIDE;
+        A.longest = P.d_counts + 6 * COUNT_STRIDE;
         HIPCHK(hipEventRecord(P.ev_el0, s));
         // the input's final count is on the device once the photon kernel is
         // done; the order is sorted there, inside the timed launch
@@ -1382,8 +1383,8 @@ static void reset_engine(omc_dev_ctx *c, int rc)
     c->finishing.clear();
     for (auto &P : c->pipes) {
         (void)hipStreamSynchronize(P.stream);
-        (void)hipMemsetAsync(P.d_counts, 0, 8 * sizeof(uint32_t), P.stream);
-        (void)hipMemsetAsync(P.d_status, 0, sizeof(DevStatus), P.stream);
+        (void)hipMemsetAsync(P.d_counts, 0, COUNT_BYTES, P.stream);
+        (void)hipMemsetAsync(P.d_status, 0, STATUS_COPIES * sizeof(DevStatus), P.stream);
         (void)hipStreamSynchronize(P.stream);
         P.cur = 0;
         P.nP = P.nE = 0;
@@ -1581,7 +1582,7 @@ const char *omc_dev_last_error(void) { return g_err; }
 static int64_t pipe_bytes(const omc_dev_ctx *c)
 {
     const size_t pb = c->precision == OMC_PREC_FP64 ? particle_bytes<double>() : particle_bytes<float>();
-    return 5 * (int64_t)pb * c->qcap + 8 * sizeof(uint32_t) + sizeof(DevStatus) + MAX_JOBS * sizeof(uint32_t) +
+    return 5 * (int64_t)pb * c->qcap + COUNT_BYTES + STATUS_COPIES * sizeof(DevStatus) + MAX_JOBS * sizeof(uint32_t) +
            MAX_SEGS * sizeof(SourceSeg) + sizeof(uint32_t) * SORT_BUCKETS * SORT_BLOCKS;
 }
 

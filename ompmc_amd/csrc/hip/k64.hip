@@ -198,17 +198,34 @@ __global__ void __launch_bounds__(256) k_gen_begin(uint32_t *counts, int nxt, ui
                                                    const uint32_t *host_segs, uint32_t *segs, int nwords)
 {
     // tails of the next queues, fetch counters, longest tracks
-    if (threadIdx.x < 8 && (threadIdx.x >= 4 || (int)(threadIdx.x & 1u) == nxt)) counts[threadIdx.x] = 0u;
+    if (threadIdx.x < 8 && (threadIdx.x >= 4 || (int)(threadIdx.x & 1u) == nxt))
+        counts[threadIdx.x * COUNT_STRIDE] = 0u;
     for (int i = threadIdx.x; i < njobs; i += blockDim.x) flags[i] = 0u;
     copy_words(segs, host_segs, nwords);
 }
 
-__global__ void __launch_bounds__(256) k_gen_end(const uint32_t *counts, const uint32_t *status, const uint32_t *flags,
-                                                 int njobs, uint32_t *host_counts, uint32_t *host_status,
+__global__ void __launch_bounds__(256) k_gen_end(const uint32_t *counts, const DevStatus *status, const uint32_t *flags,
+                                                 int njobs, uint32_t *host_counts, DevStatus *host_status,
                                                  uint32_t *host_flags)
 {
-    copy_words(host_counts, counts, 8);
-    copy_words(host_status, status, (int)(sizeof(DevStatus) / 4));
+    if (threadIdx.x < 8) host_counts[threadIdx.x] = counts[threadIdx.x * COUNT_STRIDE];
+    // the status' copies: flags or-ed, counters (the 64-bit words after the
+    // first) summed
+    constexpr int WORDS = (int)(offsetof(DevStatus, ev) / 8) + EV_N;
+    const int k = threadIdx.x;
+    if (k == 0) {
+        uint32_t over = 0, killed = 0;
+        for (int i = 0; i < STATUS_COPIES; ++i) {
+            over |= status[i].overflow;
+            killed += status[i].killed;
+        }
+        host_status->overflow = over;
+        host_status->killed = killed;
+    } else if (k < WORDS) {
+        unsigned long long v = 0;
+        for (int i = 0; i < STATUS_COPIES; ++i) v += ((const unsigned long long *)(status + i))[k];
+        ((unsigned long long *)host_status)[k] = v;
+    }
     copy_words(host_flags, flags, njobs);
 }
 
@@ -389,7 +406,7 @@ void launch_beamlet_column(const double *tally, int nslots, int nbatch, int isiz
 void launch_gen_begin(uint32_t *counts, int nxt, uint32_t *flags, int njobs, const SourceSeg *host_segs,
                       SourceSeg *segs, int nseg, hipStream_t st)
 {
-    static_assert(sizeof(SourceSeg) % 4 == 0 && sizeof(DevStatus) % 4 == 0 && sizeof(DevJob) % 4 == 0, "word copies");
+    static_assert(sizeof(SourceSeg) % 4 == 0 && sizeof(DevJob) % 4 == 0, "word copies");
     hipLaunchKernelGGL(k_gen_begin, dim3(1), dim3(256), 0, st, counts, nxt, flags, njobs, (const uint32_t *)host_segs,
                        (uint32_t *)segs, (int)(nseg * sizeof(SourceSeg) / 4));
 }
@@ -397,8 +414,8 @@ void launch_gen_begin(uint32_t *counts, int nxt, uint32_t *flags, int njobs, con
 void launch_gen_end(const uint32_t *counts, const DevStatus *status, const uint32_t *flags, int njobs,
                     uint32_t *host_counts, DevStatus *host_status, uint32_t *host_flags, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_gen_end, dim3(1), dim3(256), 0, st, counts, (const uint32_t *)status, flags, njobs,
-                       host_counts, (uint32_t *)host_status, host_flags);
+    hipLaunchKernelGGL(k_gen_end, dim3(1), dim3(256), 0, st, counts, status, flags, njobs, host_counts,
+                       host_status, host_flags);
 }
 
 void launch_job_setup(const DevJob *host_job, DevJob *job, const double *host_cdf, double *cdf, int ncdf,

@@ -59,12 +59,12 @@ void launch_probe_wait(uint32_t *flag, int us, hipStream_t st);
 // Start of a generation: zero the next generation's queue tails, both fetch
 // counters and the flags of njobs jobs, and copy the source segments from the
 // pinned host table.  counts = [photon cur/next, charged cur/next, fetch x2,
-// longest tracks x2].
+// longest tracks x2], COUNT_STRIDE words apart.
 void launch_gen_begin(uint32_t *counts, int nxt, uint32_t *flags, int njobs, const SourceSeg *host_segs,
                       SourceSeg *segs, int nseg, hipStream_t st);
 
-// End of a generation: counters, status and job flags into the pipeline's
-// pinned mirror.
+// End of a generation: counters, status (the sum of its STATUS_COPIES copies)
+// and job flags into the pipeline's pinned mirror.
 void launch_gen_end(const uint32_t *counts, const DevStatus *status, const uint32_t *flags, int njobs,
                     uint32_t *host_counts, DevStatus *host_status, uint32_t *host_flags, hipStream_t st);
 

@@ -1162,6 +1162,7 @@ __global__ void __launch_bounds__(256, Waves<R>::photon) k_photon(KArgs<R> A)
     __shared__ StageRows<R> made[RNG_LANES / 64];
     Stage<R> stage;
     stage.rows = &made[threadIdx.x >> 6];
+    A.status += blockIdx.x % STATUS_COPIES;
     events_begin<false>();
     stage_phantoms(A.phantoms, lds_ph);
     __syncthreads();
@@ -1245,13 +1246,8 @@ __global__ void __launch_bounds__(256, Waves<R>::photon) k_photon(KArgs<R> A)
         }
     }
     stage.flush(A.qe, A.status);
-    wave_max_to(A.longest, longest);
     sc.flush(G);
-    if (nyield) atomicAdd(&A.status->yields, (unsigned long long)nyield);
-    atomicAdd(&A.status->photon_steps, (unsigned long long)nsteps);
-    atomicAdd(&A.status->photon_cross, (unsigned long long)ncross);
-    atomicAdd(&A.status->photon_dep, (unsigned long long)sc.ndep);
-    events_end<false>(A.status);
+    events_end<false>(A.status, A.longest, nsteps, ncross, sc.ndep, nyield, longest);
 }
 
 template <typename R>
@@ -1259,6 +1255,7 @@ __global__ void __launch_bounds__(256, Waves<R>::electron) k_electron(KArgs<R> A
 {
     __shared__ GeoRec<R> lds_ph[MAX_PHANTOMS];
     __shared__ MedRec<R> media[MAXMED];
+    A.status += blockIdx.x % STATUS_COPIES;
     events_begin<true>();
     stage_phantoms(A.phantoms, lds_ph);
     if (threadIdx.x >= 64 && threadIdx.x < 64 + MAXMED) media[threadIdx.x - 64].stage(A.T.small->med[threadIdx.x - 64]);
@@ -1324,13 +1321,8 @@ __global__ void __launch_bounds__(256, Waves<R>::electron) k_electron(KArgs<R> A
             }
         }
     }
-    wave_max_to(A.longest, longest);
     sc.flush(G);
-    if (nyield) atomicAdd(&A.status->yields, (unsigned long long)nyield);
-    atomicAdd(&A.status->electron_steps, (unsigned long long)nsteps);
-    atomicAdd(&A.status->electron_cross, (unsigned long long)ncross);
-    atomicAdd(&A.status->electron_dep, (unsigned long long)sc.ndep);
-    events_end<true>(A.status);
+    events_end<true>(A.status, A.longest, nsteps, ncross, sc.ndep, nyield, longest);
 }
 
 }  // namespace omc
