@@ -84,21 +84,20 @@ struct SpinIdx { int i, j; };
 
 // spinRejection (ompmc.c:3097-3168)
 template <typename R>
-__device__ __forceinline__ R spin_rejection(const DevTables<R> &T, Rng &rng, int imed, int qel, R elke,
+__device__ __forceinline__ R spin_rejection(const DevTables<R> &T, const ScatRec<R> &S, Rng &rng, int imed, int qel, R elke,
                                             R beta2, R q1, R cost, bool &spin_index, bool is_single,
                                             SpinIdx &si)
 {
-    const SmallTables &S = *T.small;
     if (spin_index) {
         spin_index = false;
         R ai;
-        if (beta2 >= (R)S.b2spin_min) {
-            ai = (beta2 - (R)S.b2spin_min) * (R)S.dbeta2i;
+        if (beta2 >= S.b2spin_min) {
+            ai = (beta2 - S.b2spin_min) * S.dbeta2i;
             si.i = (int)ai;
             ai -= (R)si.i;
             si.i += OMC_MXE_SPIN + 1;
-        } else if (elke > (R)S.espml) {
-            ai = (elke - (R)S.espml) * (R)S.dleneri;
+        } else if (elke > S.espml) {
+            ai = (elke - S.espml) * S.dleneri;
             si.i = (int)ai;
             ai -= (R)si.i;
         } else {
@@ -112,7 +111,8 @@ __device__ __forceinline__ R spin_rejection(const DevTables<R> &T, Rng &rng, int
         } else {
             R qq1 = (R)2.0 * q1;
             qq1 = qq1 / ((R)1.0 + qq1);
-            R aj = qq1 * (R)S.dqq1i;
+            R aj = qq1 * S.dqq1i;
+            rounded(aj);
             si.j = (int)aj;
             if (si.j >= 15) {
                 si.j = 15;
@@ -133,7 +133,7 @@ __device__ __forceinline__ R spin_rejection(const DevTables<R> &T, Rng &rng, int
 
 // sscat (ompmc.c:3170-3199): one elastic scattering, spin rejection on
 template <typename R>
-__device__ __forceinline__ void sscat(const DevTables<R> &T, Rng &rng, int imed, int qel, R chia2, R elke, R beta2,
+__device__ __forceinline__ void sscat(const DevTables<R> &T, const ScatRec<R> &S, Rng &rng, int imed, int qel, R chia2, R elke, R beta2,
                       R &cost, R &sint)
 {
     bool spin_index = true;
@@ -143,7 +143,7 @@ __device__ __forceinline__ void sscat(const DevTables<R> &T, Rng &rng, int imed,
         xi = urand<R>(rng);
         xi = (R)2.0 * chia2 * xi / ((R)1.0 - xi + chia2);
         cost = (R)1.0 - xi;
-        rejf = spin_rejection<R>(T, rng, imed, qel, elke, beta2, (R)0, cost, spin_index, true, si);
+        rejf = spin_rejection<R>(T, S, rng, imed, qel, elke, beta2, (R)0, cost, spin_index, true, si);
         rnno = urand<R>(rng);
     } while (rnno > rejf);
     sint = m_sqrt(xi * ((R)2.0 - xi));
@@ -153,11 +153,10 @@ struct MsIdx { int i, j; };
 
 // mscat (ompmc.c:3606-3785): angle after lambda elastic mean free paths
 template <typename R>
-__device__ void mscat(const DevTables<R> &T, Rng &rng, int imed, int qel, bool &spin_index,
+__device__ void mscat(const DevTables<R> &T, const ScatRec<R> &S, Rng &rng, int imed, int qel, bool &spin_index,
                       bool &find_index, R elke, R beta2, R q1, R lambda, R chia2, R &cost, R &sint,
                       MsIdx &mi, R &omega2, SpinIdx &si)
 {
-    const SmallTables &S = *T.small;
     R xi, rejf, rnno;
     R explambda = m_exp(-lambda);
     if (lambda <= (R)13.8) {
@@ -169,7 +168,7 @@ __device__ void mscat(const DevTables<R> &T, Rng &rng, int imed, int qel, bool &
                 xi = urand<R>(rng);
                 xi = (R)2.0 * chia2 * xi / ((R)1.0 - xi + chia2);
                 cost = (R)1.0 - xi;
-                rejf = spin_rejection<R>(T, rng, imed, qel, elke, beta2, q1, cost, spin_index, false, si);
+                rejf = spin_rejection<R>(T, S, rng, imed, qel, elke, beta2, q1, cost, spin_index, false, si);
                 rnno = urand<R>(rng);
             } while (rnno > rejf);
             sint = m_sqrt(xi * ((R)2.0 - xi));
@@ -190,7 +189,7 @@ __device__ void mscat(const DevTables<R> &T, Rng &rng, int imed, int qel, bool &
                     xi = urand<R>(rng);
                     xi = (R)2.0 * chia2 * xi / ((R)1.0 - xi + chia2);
                     cosz = (R)1.0 - xi;
-                    rejf = spin_rejection<R>(T, rng, imed, qel, elke, beta2, q1, cosz, spin_index, false, si);
+                    rejf = spin_rejection<R>(T, S, rng, imed, qel, elke, beta2, q1, cosz, spin_index, false, si);
                     rnno = urand<R>(rng);
                 } while (rnno > rejf);
                 sinz = xi * ((R)2.0 - xi);
@@ -208,7 +207,7 @@ __device__ void mscat(const DevTables<R> &T, Rng &rng, int imed, int qel, bool &
     if (lambda <= (R)LAMBMAX_MS) {
         R llmbda = m_log(lambda);
         if (find_index) {
-            R ai = llmbda * (R)S.dllambi;
+            R ai = llmbda * S.dllambi;
             mi.i = (int)ai;
             ai -= (R)mi.i;
             xi = urand<R>(rng);
@@ -217,7 +216,7 @@ __device__ void mscat(const DevTables<R> &T, Rng &rng, int imed, int qel, bool &
             if (q1 < (R)QMIN_MS) {
                 mi.j = 0;
             } else if (q1 < (R)QMAX_MS) {
-                R aj = q1 * (R)S.dqmsi;
+                R aj = q1 * S.dqmsi;
                 mi.j = (int)aj;
                 aj -= (R)mi.j;
                 xi = urand<R>(rng);
@@ -248,7 +247,7 @@ __device__ void mscat(const DevTables<R> &T, Rng &rng, int imed, int qel, bool &
             xi = omega2 * u / ((R)1.0 + (R)0.5 * omega2 - u);
             if (xi > (R)1.99999) xi = (R)1.99999;
             cost = (R)1.0 - xi;
-            rejf = spin_rejection<R>(T, rng, imed, qel, elke, beta2, q1, cost, spin_index, false, si);
+            rejf = spin_rejection<R>(T, S, rng, imed, qel, elke, beta2, q1, cost, spin_index, false, si);
             rnno = urand<R>(rng);
         } while (rnno > rejf);
         sint = m_sqrt(xi * ((R)2.0 - xi));
@@ -258,7 +257,7 @@ __device__ void mscat(const DevTables<R> &T, Rng &rng, int imed, int qel, bool &
 // msdist (ompmc.c:3787-3976): PRESTA-II substeps; moves p to the step end
 // position and direction, returns the straight-line distance.
 template <typename R>
-__device__ __forceinline__ R msdist(const DevTables<R> &T, const MedRec<R> &M, Particle<R> &p, int imed, R rhof,
+__device__ __forceinline__ R msdist(const DevTables<R> &T, const ScatRec<R> &S, const MedRec<R> &M, Particle<R> &p, int imed, R rhof,
                                     R de, R tustep, R eke)
 {
     const int qel = (1 + p.iq) / 2;
@@ -301,9 +300,9 @@ __device__ __forceinline__ R msdist(const DevTables<R> &T, const MedRec<R> &M, P
     SpinIdx si = {0, 0};
     R omega2 = 0;
     R w1, sint1, cphi1, sphi1, w2, sint2, cphi2, sphi2;
-    mscat<R>(T, p.rng, imed, qel, spin_index, find_index, elke, beta2, xi, lambda, chia2, w1, sint1, mi, omega2, si);
+    mscat<R>(T, S, p.rng, imed, qel, spin_index, find_index, elke, beta2, xi, lambda, chia2, w1, sint1, mi, omega2, si);
     azimuth<R>(p.rng, cphi1, sphi1);
-    mscat<R>(T, p.rng, imed, qel, spin_index, find_index, elke, beta2, xi, lambda, chia2, w2, sint2, mi, omega2, si);
+    mscat<R>(T, S, p.rng, imed, qel, spin_index, find_index, elke, beta2, xi, lambda, chia2, w2, sint2, mi, omega2, si);
     azimuth<R>(p.rng, cphi2, sphi2);
 
     R u2 = sint2 * cphi2;
@@ -390,15 +389,14 @@ __device__ __forceinline__ void rannih(Particle<R> &a, Particle<R> &b)
 
 // brems (ompmc.c:4170-4356): a = electron (reduced energy), b = photon
 template <typename R>
-__device__ void brems(const DevTables<R> &T, Particle<R> &a, Particle<R> &b, int imed)
+__device__ void brems(const MedRec<R> &M, Particle<R> &a, Particle<R> &b)
 {
-    const MediumScalars &M = T.small->med[imed];
     const R rm = (R)RM;
     R eie = a.e, phi1, phi2;
     int l = (eie < (R)50.0) ? 1 : 3;
     int l1 = l + 1;
     R ekin = eie - rm;
-    R brmin = (R)M.ap / ekin;
+    R brmin = M.ap / ekin;
     R waux = -m_log(brmin);
     R A = a.u, B = a.v, Cc = a.w;
     R sinpsi = A * A + B * B, sindel = 0, cosdel = 0;
@@ -407,7 +405,7 @@ __device__ void brems(const DevTables<R> &T, Particle<R> &a, Particle<R> &b, int
         sindel = B / sinpsi;
         cosdel = A / sinpsi;
     }
-    R ztarg = (R)M.zbrang;
+    R ztarg = M.zbrang;
     R tteie = eie / rm;
     R beta = m_sqrt((tteie - (R)1.0) * (tteie + (R)1.0)) / tteie;
     R y2max = (R)2.0 * beta * ((R)1.0 + beta) * tteie * tteie;
@@ -421,13 +419,13 @@ __device__ void brems(const DevTables<R> &T, Particle<R> &a, Particle<R> &b, int
         br = brmin * m_exp(r6 * waux);
         esg = ekin * br;
         ese = eie - esg;
-        delta = esg / eie / ese * (R)M.delcm;
+        delta = esg / eie / ese * M.delcm;
         aux = ese / eie;
         if (delta < (R)1.0) {
-            phi1 = (R)M.dl1[l - 1] + delta * ((R)M.dl2[l - 1] + delta * (R)M.dl3[l - 1]);
-            phi2 = (R)M.dl1[l1 - 1] + delta * ((R)M.dl2[l1 - 1] + delta * (R)M.dl3[l1 - 1]);
+            phi1 = M.dl[0][l - 1] + delta * (M.dl[1][l - 1] + delta * M.dl[2][l - 1]);
+            phi2 = M.dl[0][l1 - 1] + delta * (M.dl[1][l1 - 1] + delta * M.dl[2][l1 - 1]);
         } else {
-            phi1 = (R)M.dl4[l - 1] + (R)M.dl5[l - 1] * m_log(delta + (R)M.dl6[l - 1]);
+            phi1 = M.dl[3][l - 1] + M.dl[4][l - 1] * m_log(delta + M.dl[5][l - 1]);
             phi2 = phi1;
         }
         rejf = ((R)1.0 + sq(aux)) * phi1 - (R)2.0 * aux * phi2 / (R)3.0;
@@ -487,14 +485,13 @@ __device__ void brems(const DevTables<R> &T, Particle<R> &a, Particle<R> &b, int
 // moller (ompmc.c:4359-4435).  Returns false when below the threshold (no
 // interaction, the electron simply re-enters transport).
 template <typename R>
-__device__ bool moller(const DevTables<R> &T, Particle<R> &a, Particle<R> &b, int imed)
+__device__ bool moller(const MedRec<R> &M, Particle<R> &a, Particle<R> &b)
 {
-    const MediumScalars &M = T.small->med[imed];
     const R rm = (R)RM;
     R eie = a.e, ekin = eie - rm;
     if (ekin <= (R)2.0 * (R)M.te) return false;
     R t0 = ekin / rm, e0 = t0 + (R)1.0;
-    R extrae = eie - (R)M.thmoll;
+    R extrae = eie - M.thmoll;
     R g2 = sq(t0) / sq(e0);
     R g3 = ((R)2.0 * t0 + (R)1.0) / sq(e0);
     R gmax = ((R)1.0 + (R)1.25 * g2), br, rejf4, r, r27, r28;
@@ -525,9 +522,8 @@ __device__ bool moller(const DevTables<R> &T, Particle<R> &a, Particle<R> &b, in
 
 // bhabha (ompmc.c:4438-4525): slot a keeps the higher-energy particle
 template <typename R>
-__device__ void bhabha(const DevTables<R> &T, Particle<R> &a, Particle<R> &b, int imed)
+__device__ void bhabha(const MedRec<R> &M, Particle<R> &a, Particle<R> &b)
 {
-    const MediumScalars &M = T.small->med[imed];
     const R rm = (R)RM;
     R eip = a.e, ekin = eip - rm;
     R t0 = ekin / rm, e0 = t0 + (R)1.0;

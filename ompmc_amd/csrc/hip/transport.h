@@ -693,7 +693,7 @@ __device__ __forceinline__ void electron_cutoff(const KArgs<R> &A, Particle<R> &
 // End of the ustep loop (ompmc.c:5347-5433): fictitious-cross-section
 // rejection, then the discrete interaction.
 template <typename R>
-__device__ __forceinline__ int electron_interaction(const KArgs<R> &A, Particle<R> &p, ElectronLane<R> &s)
+__device__ __forceinline__ int electron_interaction(const KArgs<R> &A, const MedRec<R> &M, Particle<R> &p, ElectronLane<R> &s)
 {
     const DevTables<R> &T = A.T;
     const int iq = p.iq;
@@ -724,16 +724,16 @@ __device__ __forceinline__ int electron_interaction(const KArgs<R> &A, Particle<
         R rnno = urand<R>(p.rng);
         if (rnno <= ebr1) {
             count_event(EV_BREMS);
-            brems<R>(T, p, b, m);
+            brems<R>(M, p, b);
             push_made_photon<R>(A, p, b);
-        } else if (p.e <= (R)T.small->med[m].thmoll) {
+        } else if (p.e <= M.thmoll) {
             if (ebr1 <= (R)0) return E_ALIVE;   // neither process possible: re-enter
             count_event(EV_BREMS);
-            brems<R>(T, p, b, m);
+            brems<R>(M, p, b);
             push_made_photon<R>(A, p, b);
         } else {
             count_event(EV_MOLLER);
-            if (moller<R>(T, p, b, m)) push<R>(A.qe, b, A.status);
+            if (moller<R>(M, p, b)) push<R>(A.qe, b, A.status);
         }
         return E_ALIVE;
     }
@@ -741,14 +741,14 @@ __device__ __forceinline__ int electron_interaction(const KArgs<R> &A, Particle<
     R rnno = urand<R>(p.rng);
     if (rnno < pbr1) {
         count_event(EV_BREMS);
-        brems<R>(T, p, b, m);
+        brems<R>(M, p, b);
         push_made_photon<R>(A, p, b);
         return E_ALIVE;
     }
     R pbr2 = s.elke * eb.br21 + eb.br20;
     if (rnno < pbr2) {
         count_event(EV_BHABHA);
-        bhabha<R>(T, p, b, m);
+        bhabha<R>(M, p, b);
         push<R>(A.qe, b, A.status);
         return E_ALIVE;
     }
@@ -805,7 +805,7 @@ __device__ __forceinline__ int zero_ustep(const KArgs<R> &A, const MedRec<R> &M,
 }
 
 template <typename R>
-__device__ __forceinline__ int electron_iteration(const KArgs<R> &A, const MedRec<R> *media, Particle<R> &p,
+__device__ __forceinline__ int electron_iteration(const KArgs<R> &A, const ElectronRec<R> &rec, Particle<R> &p,
                                                   ElectronLane<R> &s, ElectronGeo<R> &G, Scorer<R> &sc,
                                                   uint32_t &nsteps, uint32_t &ncross)
 {
@@ -823,7 +823,7 @@ __device__ __forceinline__ int electron_iteration(const KArgs<R> &A, const MedRe
         if (eie <= G.g->ecut[s.imed + 1]) { electron_cutoff<R>(A, p, G, sc, eie); return E_DONE; }
         s.phase = 1;
     }
-    const MedRec<R> &M = media[max(s.imed, 0)];
+    const MedRec<R> &M = rec.med[max(s.imed, 0)];
     if (s.phase != 2) {
         s.compute_tstep = 1;
         s.eke = eie - rm;
@@ -985,7 +985,7 @@ __device__ __forceinline__ int electron_iteration(const KArgs<R> &A, const MedRe
             // after ausgab, which scores in the pre-step region
             Particle<R> q = p;
             count_lane_event(EV_MSDIST);
-            ustep = msdist<R>(T, M, q, imed, rhof, de, tustep, s.eke);
+            ustep = msdist<R>(T, rec.scat, M, q, imed, rhof, de, tustep, s.eke);
             p.rng = q.rng;
             xf = q.x; yf = q.y; zf = q.z; uf = q.u; vf = q.v; wf = q.w;
             if (ustep < (R)0) ustep = (R)0.0;
@@ -1009,7 +1009,7 @@ __device__ __forceinline__ int electron_iteration(const KArgs<R> &A, const MedRe
             s.phase = 1;
             return E_ALIVE;
         }
-        return electron_interaction<R>(A, p, s);
+        return electron_interaction<R>(A, M, p, s);
     }
     R edep = de;
     R ekef = s.eke - de;
@@ -1026,7 +1026,7 @@ __device__ __forceinline__ int electron_iteration(const KArgs<R> &A, const MedRe
             R etap = elkems * ebs.eta1 + ebs.eta0;
             chia2 *= etap;
             count_lane_event(EV_SSCAT);
-            sscat<R>(T, p.rng, imed, qel, chia2, elkems, beta2, costhe, sinthe);
+            sscat<R>(T, rec.scat, p.rng, imed, qel, chia2, elkems, beta2, costhe, sinthe);
         } else {
             sinthe = (R)0.0;
             costhe = (R)1.0;
@@ -1063,7 +1063,7 @@ __device__ __forceinline__ int electron_iteration(const KArgs<R> &A, const MedRe
     if (total_tstep < 1.0E-9) s.demfp = (R)0.0;
     if (s.demfp >= (R)EPSEMFP) return zero_ustep<R>(A, M, p, s, G, sc, b, nsteps, ncross);
 
-    return electron_interaction<R>(A, p, s);
+    return electron_interaction<R>(A, M, p, s);
 }
 
 // ============================================================ kernels =====
@@ -1254,11 +1254,11 @@ template <typename R>
 __global__ void __launch_bounds__(256, Waves<R>::electron) k_electron(KArgs<R> A)
 {
     __shared__ GeoRec<R> lds_ph[MAX_PHANTOMS];
-    __shared__ MedRec<R> media[MAXMED];
+    __shared__ ElectronRec<R> rec;
     A.status += blockIdx.x % STATUS_COPIES;
     events_begin<true>();
     stage_phantoms(A.phantoms, lds_ph);
-    if (threadIdx.x >= 64 && threadIdx.x < 64 + MAXMED) media[threadIdx.x - 64].stage(A.T.small->med[threadIdx.x - 64]);
+    rec.stage(*A.T.small);
     __syncthreads();
     Particle<R> p;
     ElectronLane<R> s;
@@ -1301,7 +1301,7 @@ __global__ void __launch_bounds__(256, Waves<R>::electron) k_electron(KArgs<R> A
             in_end >= A.drain_min && __ballot(exhausted) != 0 && (uint32_t)__popcll(live) <= A.drain_lanes;
         ring_fill(p.rng, alive, live);
         if (alive) {
-            int r = electron_iteration<R>(A, media, p, s, G, sc, nsteps, ncross);
+            int r = electron_iteration<R>(A, rec, p, s, G, sc, nsteps, ncross);
             ++trips;
             ++here;
             if (r != E_DONE && trips > MAX_ITERS) {     // watchdog: no particle runs forever
