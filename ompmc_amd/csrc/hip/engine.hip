@@ -81,7 +81,7 @@ constexpr size_t RESULT_KEEP = 32u << 20;   // result buffers up to this size ar
 constexpr int RESULT_BUFFERS = 2;
 // Pipelines of a context that names no number: one per hardware queue, at
 // least 4 and at most 6.  With HIP's default of 4 queues (ms, 4 / 6
-// pipelines): FP32 slab of 1e8 histories 324-358 / 346, 400 beamlets 458 /
+// pipelines, when the rule was made; the kernels have become faster since): FP32 slab of 1e8 histories 324-358 / 346, 400 beamlets 458 /
 // 479, five-beam plan 190 / 223, serving burst 141 / 156, 1e6 photons on a
 // graded grid 29 / 42, 5e6 FP64 slab histories 68 / 93: a pipeline that shares
 // a queue runs after the other one.  With 16 queues the FP32 engine gains up
@@ -922,7 +922,7 @@ static int admit_works(omc_dev_ctx *c, bool &fresh)
         J.nhist = jn;
         J.batch = split ? w->next_batch : -1;
         // serving requests share each refill in slices of chunk/8 (spreading
-        // a 6.5e5-history request over all six pipelines instead raised the
+        // a 6.5e5-history request over all of six pipelines instead raised the
         // FP32 p50 of the latency stream from 57 to 69-77 ms); a synchronous
         // run spreads its histories over all pipelines
         const int64_t npipes = (int64_t)c->pipes.size();

@@ -1099,8 +1099,8 @@ template <typename R> __device__ __forceinline__ uint32_t trips_per_launch(const
 // particles and rings allows; 4 spills registers and measures the same) /
 // electron 4 (128 VGPRs and a few spills; alone on the device 3 waves without
 // spills are faster, 81.3 against 84.3 ms per 2e7 histories, but with four
-// pipelines on it a slab of 1e8 takes 340 ms with 3 and 324 with 4), FP64 photon 2 / electron 2 (a few spills, still faster than one
-// wave).
+// pipelines on it a slab of 1e8 took 340 ms with 3 and 324 with 4), FP64 photon
+// 2 / electron 2 (a few spills, still faster than one wave: 52 against 61 ms).
 #ifndef OMC_WAVES_P32
 #define OMC_WAVES_P32 3
 #endif
@@ -1122,7 +1122,8 @@ template <> struct Waves<double> { static constexpr int photon = OMC_WAVES_P64, 
 // its lanes as they come free; towards the end only what its lanes need.  All
 // wavefronts of the device add to this one counter, which serves an atomic
 // every 11 to 12 ns.  Photon / charged-particle kernel on 2e7 FP32 slab
-// histories, ms: no chunks 20.9 / 88.3, 16 20.7 / 87.2, 32 18.5 / 85.3, 64
+// histories, ms, while the counter shared its line with the queue tails (9.5 /
+// 75.9 now, with 64 and 32): no chunks 20.9 / 88.3, 16 20.7 / 87.2, 32 18.5 / 85.3, 64
 // 16.2 / 88.4, 128 16.7 / 110, 256 21 / 176: a charged-particle launch reads
 // its longest tracks first, and a large share keeps too many of them in one
 // wavefront.
