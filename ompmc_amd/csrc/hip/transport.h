@@ -693,9 +693,13 @@ __device__ __forceinline__ void electron_cutoff(const KArgs<R> &A, Particle<R> &
 // End of the ustep loop (ompmc.c:5347-5433): fictitious-cross-section
 // rejection, then the discrete interaction.
 template <typename R>
-__device__ __forceinline__ int electron_interaction(const KArgs<R> &A, const MedRec<R> &M, Particle<R> &p, ElectronLane<R> &s)
+__device__ __forceinline__ int electron_interaction(const KArgs<R> &A, const ElectronRec<R> &rec, Particle<R> &p,
+                                                    ElectronLane<R> &s)
 {
     const DevTables<R> &T = A.T;
+    // (of the medium the particle is in now: after a step through vacuum that
+    // is not the one the iteration began in)
+    const MedRec<R> &M = rec.med[s.imed];
     const int iq = p.iq;
     const int qel = (1 + iq) / 2;
     // ---- end of the ustep loop: fictitious-cross-section rejection ----
@@ -1009,7 +1013,7 @@ __device__ __forceinline__ int electron_iteration(const KArgs<R> &A, const Elect
             s.phase = 1;
             return E_ALIVE;
         }
-        return electron_interaction<R>(A, M, p, s);
+        return electron_interaction<R>(A, rec, p, s);
     }
     R edep = de;
     R ekef = s.eke - de;
@@ -1063,7 +1067,7 @@ __device__ __forceinline__ int electron_iteration(const KArgs<R> &A, const Elect
     if (total_tstep < 1.0E-9) s.demfp = (R)0.0;
     if (s.demfp >= (R)EPSEMFP) return zero_ustep<R>(A, M, p, s, G, sc, b, nsteps, ncross);
 
-    return electron_interaction<R>(A, M, p, s);
+    return electron_interaction<R>(A, rec, p, s);
 }
 
 // ============================================================ kernels =====
