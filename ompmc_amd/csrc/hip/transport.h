@@ -1013,7 +1013,11 @@ __device__ __forceinline__ int electron_iteration(const KArgs<R> &A, const Elect
             s.phase = 1;
             return E_ALIVE;
         }
-        return electron_interaction<R>(A, rec, p, s);
+        const int r = electron_interaction<R>(A, rec, p, s);
+        // the energy bin may be another medium's (the last in which the tstep
+        // loop began, with a step of length 0): after a rejection it is found anew
+        if (s.phase == 3) s.phase = 1;
+        return r;
     }
     R edep = de;
     R ekef = s.eke - de;
