@@ -973,7 +973,9 @@ __device__ __forceinline__ int electron_iteration(const KArgs<R> &A, const Elect
         howfar<R>(b, p.x, p.y, p.z, p.u, p.v, p.w, side, ustep);
     }
     if (ustep < (R)0) ustep = (R)0.0;
-    bool no_step = ustep == (R)0.0 || imed == -1;
+    // (a multiple-scattering step draws its numbers at length 0 too, where the
+    // skin depth is negative)
+    bool no_step = (ustep == (R)0.0 && !called_msdist) || imed == -1;
     const R rhof = s.rhof;
     R vstep = ustep;
     if (!no_step) {
