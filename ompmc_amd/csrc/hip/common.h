@@ -228,6 +228,16 @@ __device__ __forceinline__ uint32_t wave_reserve(uint32_t *counter, uint32_t n_p
     return base + lanes_below(m) * n_per_lane;
 }
 
+// Between LDS accesses of lanes of one wavefront to each other's words.  LDS
+// executes a wavefront's accesses in order; this keeps the compiler to it (no
+// instruction).
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Tops up the Philox rings of a wavefront's live lanes; every lane of the
 // wavefront calls it, converged (`mask` is the ballot of `live`).
 //
@@ -249,6 +259,7 @@ __device__ __forceinline__ uint32_t wave_reserve(uint32_t *counter, uint32_t n_p
 #endif
 __device__ __forceinline__ void ring_fill(Rng &r, bool live, uint64_t mask)
 {
+    wave_lds_fence();                  // the owners' reads so far before the helpers' writes
     const uint32_t cur = r.ctr >> 2;
     uint32_t tb = max(r.tail >> 2, cur);                    // first block not in the ring
     uint32_t room = live ? cur + RNG_RING - tb : 0u;
@@ -284,11 +295,7 @@ __device__ __forceinline__ void ring_fill(Rng &r, bool live, uint64_t mask)
         }
     }
     if (live) r.tail = tb << 2;
-    // the helpers' writes come before the owners' reads: LDS executes a
-    // wavefront's accesses in order, and this keeps the compiler to it
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_lds_fence();                  // the helpers' writes before the owners' reads
 }
 
 // ------------------------------------------------------------- layouts ----

@@ -298,6 +298,7 @@ template <typename R> struct Stage {
     __device__ __forceinline__ void flush(const Queue<R> &q, DevStatus *st)
     {
         if (n == 0) return;
+        wave_lds_fence();              // rows written by other lanes before they are read
         const uint32_t lane = (uint32_t)lane_id();
         uint32_t base = 0;
         if (lane == 0) base = atomicAdd(q.count, n);
@@ -314,6 +315,7 @@ template <typename R> struct Stage {
             }
         }
         n = 0;
+        wave_lds_fence();              // and read before other lanes write them again
     }
     __device__ __forceinline__ void push(const Queue<R> &q, bool have, const Particle<R> &p, DevStatus *st)
     {
