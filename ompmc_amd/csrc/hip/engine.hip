@@ -810,11 +810,9 @@ template <typename R> static int upload_phantom(omc_dev_ctx *c, const omc_phanto
 }
 
 // -------------------------------------------------------------- scheduler --
-// Bytes of a job's pooled buffer: its grids and, at the end, its spectrum.
-static size_t job_bytes(size_t tally_bytes)
-{
-    return ((tally_bytes + 255) & ~(size_t)255) + 2 * OMC_INVDIM * sizeof(double);
-}
+// Bytes of a job's pooled buffer: its grids and behind them its spectrum (both
+// doubles).  Admission checks the budget for exactly these (work_bytes).
+static size_t job_bytes(size_t tally_bytes) { return tally_bytes + 2 * OMC_INVDIM * sizeof(double); }
 
 static void release_job(omc_dev_ctx *c, int j)
 {
@@ -849,9 +847,9 @@ static size_t work_bytes(const Work *w)
 {
     if (w->scratch) return 0;
     if (w->split_k)   // the next batch's grid, spectrum and ledger, and the sums with the first batch
-        return sizeof(double) * (size_t)w->nreg * (w->acc ? 1 : 3) + 2 * OMC_INVDIM * sizeof(double) +
+        return job_bytes(sizeof(double) * (size_t)w->nreg) + (w->acc ? 0 : 2 * sizeof(double) * (size_t)w->nreg) +
                (w->ledger ? sizeof(double) * OMC_LEDGER * (size_t)w->nperbatch : 0);
-    return sizeof(double) * (size_t)w->nreg * w->slots + 2 * OMC_INVDIM * sizeof(double) +
+    return job_bytes(sizeof(double) * (size_t)w->nreg * w->slots) +
            (w->ledger ? sizeof(double) * OMC_LEDGER * (size_t)w->nhist : 0);
 }
 
@@ -903,7 +901,7 @@ static int admit_works(omc_dev_ctx *c, bool &fresh)
         } else if (!rc) {
             // grids and spectrum in one buffer of the pool
             rc = pool_alloc(c, (void **)&J.tally, job_bytes(J.tally_bytes));
-            if (!rc) J.cdf = (double *)((char *)J.tally + job_bytes(J.tally_bytes)) - 2 * OMC_INVDIM;
+            if (!rc) J.cdf = (double *)((char *)J.tally + J.tally_bytes);
         }
         if (!rc && w->ledger) {
             J.ledger_bytes = sizeof(double) * OMC_LEDGER * (size_t)jn;
