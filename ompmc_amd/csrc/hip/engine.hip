@@ -89,7 +89,9 @@ constexpr int RESULT_BUFFERS = 2;
 // exercised at 6; the autotuner reaches 10-12 where a workload gains.
 constexpr int LEAST_PIPES = 4;
 constexpr int DEFAULT_PIPES = 6;
-constexpr int PROBE_US = 150;         // longest wait of the overlap probe
+constexpr int PROBE_US = 150;         // wait of the overlap probe...
+constexpr int PROBE_US_MOST = 9600;   // ...and at most, where other work delays it
+constexpr int PROBE_SLACK_US = 150;   // launch and wait for the two kernels behind it (some 30 us)
 constexpr int PROBE_MISSES = 8;       // streams in a row without a queue of their own that end the search
 constexpr int64_t DEFAULT_CHUNK = 1 << 22;
 // Batches of one work admitted batch by batch that may be in flight at once
@@ -407,21 +409,28 @@ template <typename R> Queue<R> queue_view(const omc_dev_ctx *c, const Pipe &P, i
 // bounded time) for one on `b`, launched after it.  That one follows another on
 // `b`, so it is held back behind everything earlier in its hardware queue (two
 // streams' kernels may overlap within a queue while neither waits for one of
-// its own stream).
+// its own stream).  Behind `a` in its queue, `b` is done as soon as the wait is
+// over; later than that, it was other work on the device that held it up (that
+// of another context, say), and a longer wait decides.  Without that a context
+// made while another one was running found 4 streams instead of 6.
 int streams_overlap(omc_dev_ctx *c, hipStream_t a, hipStream_t b, bool *yes)
 {
-    uint32_t seen = 0;
-    launch_set_u32(c->d_probe, 2, 0u, a);
-    HIPCHK(hipStreamSynchronize(a));
-    launch_probe_wait(c->d_probe, PROBE_US, a);
-    launch_set_u32(c->d_probe, 1, 0u, b);
-    launch_set_u32(c->d_probe, 1, 1u, b);
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(b));
-    HIPCHK(hipMemcpyAsync(&seen, c->d_probe + 1, sizeof seen, hipMemcpyDeviceToHost, a));
-    HIPCHK(hipStreamSynchronize(a));
-    *yes = seen != 0;
-    return OMC_OK;
+    for (int us = PROBE_US;; us = std::min(4 * us, PROBE_US_MOST)) {
+        uint32_t seen = 0;
+        launch_set_u32(c->d_probe, 2, 0u, a);
+        HIPCHK(hipStreamSynchronize(a));
+        const double t0 = now_ms(c);
+        launch_probe_wait(c->d_probe, us, a);
+        launch_set_u32(c->d_probe, 1, 0u, b);
+        launch_set_u32(c->d_probe, 1, 1u, b);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipStreamSynchronize(b));
+        const double took = now_ms(c) - t0;
+        HIPCHK(hipMemcpyAsync(&seen, c->d_probe + 1, sizeof seen, hipMemcpyDeviceToHost, a));
+        HIPCHK(hipStreamSynchronize(a));
+        *yes = seen != 0;
+        if (*yes || us == PROBE_US_MOST || took < 1.0E-3 * (us + PROBE_SLACK_US)) return OMC_OK;
+    }
 }
 
 // Streams for `most` pipelines.  The runtime maps streams onto a few hardware
