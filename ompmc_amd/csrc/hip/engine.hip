@@ -1211,14 +1211,20 @@ static int pull_segments(omc_dev_ctx *c, int pi, int64_t room, uint32_t &injP, u
 }
 
 // Blocks of a transport launch over at most n particles.  No launch takes
-// more than 15/16 of the blocks the device holds resident: blocks beyond that
-// would only wait, and the other pipelines' small kernels (counters, flags,
-// copies, source) would wait behind them for a slot, up to 3.6 ms each
-// (serving burst 137 ms with twice the resident blocks, 129 with 15/16; FP32
-// slab of 1e8 histories 318 and 311).  A small launch spreads over SPREAD_WAVES
-// wavefronts per SIMD, or over its share of the device where other pipelines
-// are at work too (1e6 photons on a graded grid 30.5 ms without sharing, 27.9
-// with; 5e6 FP64 slab histories 66.6 and 64.3).
+// more than 15/16 of the charged-particle blocks the device holds resident:
+// blocks beyond that would only wait, and the other pipelines' small kernels
+// (counters, flags, copies, source) would wait behind them for a slot, up to
+// 3.6 ms each (serving burst 137 ms with twice the resident blocks, 129 with
+// 15/16; FP32 slab of 1e8 histories 318 and 311).  FP32 photon launches go by
+// the same number although the device holds a quarter less of theirs: with
+// 15/16 of their own, ms against these, the slab takes 287.5 against 282.2,
+// 400 beamlets 386 against 380, the serving burst 121 against 116, the five-beam
+// plan 178 against 165.  A small launch spreads over SPREAD_WAVES wavefronts
+// per SIMD, or over its share of the device where other pipelines are at work
+// too (1e6 photons on a graded grid 30.5 ms without sharing, 27.9 with; 5e6
+// FP64 slab histories 66.6 and 64.3).  The share counts the pipelines at work
+// when the launch is made: of several that start in one turn the first takes
+// its width as if alone.
 static int transport_grid(const omc_dev_ctx *c, int64_t n)
 {
     int active = 0;
