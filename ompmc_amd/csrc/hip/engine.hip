@@ -319,6 +319,7 @@ struct omc_dev_ctx {
     struct ResultBuf { double *p; int64_t cap; };
     std::vector<ResultBuf> results;   // free ones
     int64_t result_cap = 0;           // regions they have room for (0: none are kept)
+    int results_made = 0;             // buffers of that size made so far, at most RESULT_BUFFERS
     // job set-up
     struct JobStage { DevJob job; double cdf[2 * OMC_INVDIM]; };
     JobStage *h_stage = nullptr;      // [JOB_STAGES] pinned
@@ -728,16 +729,8 @@ static int grow_finish_scratch(omc_dev_ctx *c, int64_t nvox)
     c->fin_nvox = nvox;
     for (auto &r : c->results) (void)hipHostFree(r.p);
     c->results.clear();
-    c->result_cap = 0;
-    if (sums <= RESULT_KEEP) {
-        for (int i = 0; i < RESULT_BUFFERS; ++i) {
-            double *r = nullptr;
-            if (hipHostMalloc((void **)&r, sums, hipHostMallocDefault) != hipSuccess)
-                return fail(OMC_EDEVICE, "pinned result buffers (%zu bytes)", sums);
-            c->results.push_back({ r, nvox + 1 });
-        }
-        c->result_cap = nvox + 1;
-    }
+    c->results_made = 0;
+    c->result_cap = sums <= RESULT_KEEP ? nvox + 1 : 0;
     return OMC_OK;
 }
 
@@ -1011,6 +1004,20 @@ static double *sums_target(omc_dev_ctx *c, Work *w)
         return w->res;
     }
     return c->h_sums;
+}
+
+// A pinned result buffer more where more requests are on their way than buffers
+// are free: only programs that submit requests pay for them, and pinning runs
+// beside the device's work.  Where it fails, vectors take the results.
+static void make_result_buffer(omc_dev_ctx *c)
+{
+    if (!c->result_cap || c->results_made == RESULT_BUFFERS || c->unfinished <= (int)c->results.size()) return;
+    c->results_made++;
+    double *p = nullptr;
+    if (hipHostMalloc((void **)&p, 2 * sizeof(double) * (size_t)c->result_cap, hipHostMallocDefault) == hipSuccess)
+        c->results.push_back({ p, c->result_cap });
+    else
+        (void)hipGetLastError();
 }
 
 // Gives a request's result buffer back (one that was made for smaller
@@ -1436,6 +1443,7 @@ template <typename R> static int turn(omc_dev_ctx *c)
     bool any = !c->finishing.empty();
     for (auto &P : c->pipes) any |= P.inflight;
     if (!any) return 0;
+    make_result_buffer(c);
     int spins = 0;
     for (;;) {
         if (!c->finishing.empty()) {
