@@ -247,10 +247,11 @@ __device__ __forceinline__ void wave_lds_fence()
 // particle's trip spent a fifth of its time on four or five passes of one
 // lane each.
 //
-// A fuller wavefront computes one block per lane and pass, as long as
-// RNG_FILL_LANES lanes have room for one or a lane holds fewer than
-// RNG_FILL_MIN: the few lanes that drew most in the last trip catch up over
-// the next ones instead of costing the wavefront a pass each.
+// In a fuller wavefront each lane computes its own, two blocks a pass (one
+// where it has room for one only), as long as RNG_FILL_LANES lanes have room
+// for two or a lane holds fewer than RNG_FILL_MIN: the few lanes that drew most
+// in the last trip catch up over the next ones instead of costing the wavefront
+// a pass each.
 #ifndef OMC_RNG_FILL_LANES
 #define OMC_RNG_FILL_LANES 24
 #endif

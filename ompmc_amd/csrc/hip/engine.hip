@@ -77,16 +77,24 @@ constexpr int MAX_SEGS = 512;
 constexpr size_t COUNT_BYTES = 8 * COUNT_STRIDE * sizeof(uint32_t);
 constexpr int MAX_PIPES = 16;
 constexpr int JOB_STAGES = 64;        // jobs set up before the host waits for the set-ups
-constexpr size_t RESULT_KEEP = 32u << 20;   // result buffers up to this size are kept pinned
+// Result buffers of requests kept pinned: two, of up to 32 MiB each, so that a
+// context holds at most 64 MiB of them.  Burst of 12 requests, ms, with 0 / 1 /
+// 2 / 4 buffers: 130 / 127 / 119 / 120; one request at a time on the
+// 128x128x96 patient (24 MiB) 17.8 with none, 14.5 with one.  Above the limit
+// the sums go through ordinary memory: on 256x256x160 voxels (160 MiB) 70.5 ms a
+// request, where buffers of that size would take 32.
+constexpr size_t RESULT_KEEP = 32u << 20;
 constexpr int RESULT_BUFFERS = 2;
 // Pipelines of a context that names no number: one per hardware queue, at
-// least 4 and at most 6.  With HIP's default of 4 queues (ms, 4 / 6
-// pipelines, when the rule was made; the kernels have become faster since): FP32 slab of 1e8 histories 324-358 / 346, 400 beamlets 458 /
-// 479, five-beam plan 190 / 223, serving burst 141 / 156, 1e6 photons on a
-// graded grid 29 / 42, 5e6 FP64 slab histories 68 / 93: a pipeline that shares
-// a queue runs after the other one.  With 16 queues the FP32 engine gains up
-// to 10 pipelines and FP64 is flat from 6 on, but the serving loop has been
-// exercised at 6; the autotuner reaches 10-12 where a workload gains.
+// least 4 and at most 6.  With HIP's default of 4 queues a fifth and sixth
+// pipeline share a queue with another and run after it (ms, 4 / 6 pipelines):
+// FP32 slab of 1e8 histories 286 / 302, of 4e6 31 / 51, 400 beamlets 400 / 417,
+// serving burst 117 / 135, 1e6 electrons 64 / 97, 1e6 photons on a graded grid
+// 25 / 43, 5e6 FP64 slab histories 60 / 91; up to 1e5 histories, which one or two
+// pipelines hold, the same.  With 16 queues the FP32 engine gains up to 10
+// pipelines (slab 3.39e8 histories/s with 6, 3.49e8 with 10) and FP64 is flat
+// from 6 on, but the serving loop has been exercised at 6; the autotuner
+// reaches 10-12 where a workload gains.
 constexpr int LEAST_PIPES = 4;
 constexpr int DEFAULT_PIPES = 6;
 constexpr int PROBE_US = 150;         // wait of the overlap probe...
@@ -102,15 +110,19 @@ constexpr int64_t MAX_SPLIT_INFLIGHT = 16;
 constexpr uint32_t DEFAULT_YIELD_TRIPS = 4096;
 // Particles x trips of a launch of middling size (trips_per_launch): it cannot
 // fill the device and hands its particles on early.  A generation costs
-// 0.2-0.5 ms.  ms at 512 trips / 2^24 / 2^23 / 2^22 particle-trips: 1e6 photons
-// on the graded 61^3 grid 27.9 / 28.0 / 26.7 / 26.4, 2e5 electrons 38.4 / 36.5 /
-// 37.6 / 35.0, 5e6 FP64 slab histories 64.3 / 65.3 / 63.1 / 65.1, 25 FP64
-// beamlets 47.3 / 48.3 / 46.2 / 48.5.
+// 0.2-0.5 ms.  ms at 2^20 / 2^23 / 2^26 particle-trips / no early hand-on:
+//   6 MeV electrons, FP32    6.4e4 26.3 / 26.9 / 27.9 / 28.0   2.6e5 36.5 / 37.3 / 49.8 / 49.5   1e6 63.3 / 64.3 / 65.9 / 77.8
+//   slab, FP32               1e5 14.7 / 13.6 / 13.9 / 14.5     1e6 23.5 / 22.6 / 25.4 / 26.0     4e6 31.9 / 31.2 / 33.7 / 35.8
+//   slab, FP64               1e5 22.3 / 24.3 / 24.8 / 26.9     1e6 36.0 / 35.5 / 38.9 / 40.0     4e6 57.8 / 56.1 / 55.7 / 60.2
+// and below that all the same (four or fewer particles to a wavefront).
 constexpr uint32_t SMALL_TRIPS = 1u << 23;
 // Wavefronts per SIMD over which a small launch's particles are spread
 // (lanes_used) while it is the only one.  A 1e3-photon FP64 call on the 40^3
-// water cube takes 8.7 ms with 64 particles to a wavefront, 5.1-5.3 ms spread
-// over 1, 2 or 4 per SIMD; the FP32 beamlet request 22.5 ms against 18.7.
+// water cube takes 8.7 ms with 64 particles to a wavefront, 4.3-4.7 spread
+// over 1, 2 or 4 per SIMD; the FP32 beamlet request 22.5 against 13.  Between
+// 1, 2 and 4 (ms): 1.6e4 6 MeV electrons 20.8 / 21.3 / 23.4, 2e5 32.2 / 34.0 /
+// 35.3, 2.6e5 36.4 / 37.3 / 41.1; photons from 1e3 to 4e6 in either precision
+// within 3%; beamlet request 13.3 / 12.7 / 12.9.
 constexpr int SPREAD_WAVES = 2;
 // Drain compaction: once a launch's input is used up, a wavefront with at
 // most 32 live lanes hands its particles (after 16 trips in the launch) to

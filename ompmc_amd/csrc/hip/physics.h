@@ -44,8 +44,11 @@ template <typename R> __device__ __forceinline__ R sq(R x) { return x * x; }
 
 // A product that is rounded before it is used.  The FP32 build fuses a
 // multiplication with the addition it feeds wherever the compiler finds the
-// two in one block; where that depends on the code around them, this fixes
-// the choice, so that changes around it do not change the histories.
+// two in one block.  This fixes the choice at the products where a change of
+// the code around them had changed it, found by comparing sums and event
+// counts; every other product is the compiler's, so FP32 histories may change
+// in the last bit with the compiler or the code (FP64, built without fusing,
+// replays the CPU restatement).
 template <typename R> __device__ __forceinline__ void rounded(R &x) { asm volatile("" : "+v"(x)); }
 
 // pwlfInterval / pwlfEval (ompmc.c:203-211)
