@@ -95,6 +95,7 @@ constexpr int RESULT_BUFFERS = 2;
 // pipelines (slab 3.39e8 histories/s with 6, 3.49e8 with 10) and FP64 is flat
 // from 6 on, but the serving loop has been exercised at 6; the autotuner
 // reaches 10-12 where a workload gains.
+constexpr int HIP_DEFAULT_QUEUES = 4;
 constexpr int LEAST_PIPES = 4;
 constexpr int DEFAULT_PIPES = 6;
 constexpr int PROBE_US = 150;         // wait of the overlap probe...
@@ -446,17 +447,29 @@ int streams_overlap(omc_dev_ctx *c, hipStream_t a, hipStream_t b, bool *yes)
     }
 }
 
+// Hardware queues the runtime has streams share (it reads the variable once, at
+// its start).
+int hw_queues()
+{
+    const char *q = getenv("GPU_MAX_HW_QUEUES");
+    const int n = q ? atoi(q) : 0;
+    return n > 0 ? n : HIP_DEFAULT_QUEUES;
+}
+
 // Streams for `most` pipelines.  The runtime maps streams onto a few hardware
 // queues (GPU_MAX_HW_QUEUES, 4 unless set) by its own count of their users,
 // and two pipelines on one queue run in turn.  Streams that overlap all those
-// chosen before are taken as long as the runtime gives some; the rest, up to
-// `least`, share.  The streams passed over stay until the end, so that the
-// next ones land on other queues.
+// chosen before are taken, no more than there are queues, as long as the
+// runtime gives some; the rest, up to `least`, share.  The streams passed over
+// stay until the end, so that the next ones land on other queues.  Looking for
+// a fifth queue where there are four took 9 of the 12 ms of making a context
+// (8 streams made, probed and destroyed).
 int pick_streams(omc_dev_ctx *c, int least, int most, std::vector<hipStream_t> &out)
 {
     std::vector<hipStream_t> passed;
     int rc = OMC_OK;
-    for (int misses = 0; !rc && (int)out.size() < most && misses < PROBE_MISSES;) {
+    const int apart_most = std::min(most, hw_queues());
+    for (int misses = 0; !rc && (int)out.size() < apart_most && misses < PROBE_MISSES;) {
         hipStream_t s = nullptr;
         if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) { rc = fail(OMC_EDEVICE, "stream"); break; }
         bool apart = true;
