@@ -91,10 +91,9 @@ constexpr int RESULT_BUFFERS = 2;
 // FP32 slab of 1e8 histories 286 / 302, of 4e6 31 / 51, 400 beamlets 400 / 417,
 // serving burst 117 / 135, 1e6 electrons 64 / 97, 1e6 photons on a graded grid
 // 25 / 43, 5e6 FP64 slab histories 60 / 91; up to 1e5 histories, which one or two
-// pipelines hold, the same.  With 16 queues the FP32 engine gains up to 10
-// pipelines (slab 3.39e8 histories/s with 6, 3.49e8 with 10) and FP64 is flat
-// from 6 on, but the serving loop has been exercised at 6; the autotuner
-// reaches 10-12 where a workload gains.
+// pipelines hold, the same.  With 16 queues both engines are flat from 4 to 12
+// pipelines on the slab (FP32 3.34e8-3.50e8 histories/s, FP64 1.38e8-1.40e8,
+// two runs differ by 2%); 6 is what the serving loop has been exercised at.
 constexpr int HIP_DEFAULT_QUEUES = 4;
 constexpr int LEAST_PIPES = 4;
 constexpr int DEFAULT_PIPES = 6;
