@@ -39,7 +39,7 @@ with D.Engine(1) as eng:
     eng.upload_media(pp.tab)
     pid = eng.upload_phantom(pp.ph, pp.reg)
     for k in range(8):
-        run = threading.Thread(target=lambda: eng.run_dosxyz(pid, pp.src, 40000000, 10, nreg=pp.reg.nreg))
+        run = threading.Thread(target=lambda: eng.run_dosxyz(pid, pp.src, 80000000, 10, nreg=pp.reg.nreg))
         run.start()
         time.sleep(0.02 + 0.01 * k)
         running = []
